@@ -12,7 +12,10 @@
 // states the quantiser).
 //
 // The plain and grouped GEMM entry points (bf16 activations, no workspace) run the same tiles, the activations
-// quantised into hi + lo rows while they are staged.
+// quantised into hi + lo rows while they are staged.  They are HBM-bound where experts have few rows: 2,000 Zipf-routed
+// rows over a raw store, gate_up and down, 1,390 -> 536 us (1.7 GB; bit-identical) when the scales went through LDS
+// instead of scattered byte loads, tiles stopped staging and multiplying their empty 16-row blocks, column groups got
+// the XCD order, and the kernels, 400 registers before, came to fit two workgroups per CU.
 //
 // Weight layouts (template W): the store's raw and PS4 slots (row r: 1,440 code bytes, then a raw 90-byte or PS4
 // 46-byte scale row; lane (q, n) reads the 16 bytes of group 4t + q of row n, already the MFMA's B order) and the t950
@@ -35,23 +38,6 @@ struct WSrc {
   const uint8_t* codes;     // raw/PS4: row 0's code bytes (row pitch 1,440); t950: block 0 of the matrix
   const uint8_t* scales;    // raw/PS4: row 0's scale row (pitch 90 or 46); t950: unused
 };
-
-// Store layouts (raw, PS4): the 16 code bytes of (row n, group 4t + q) of row block rblk for lane 16 q + n, and that
-// group's E8M0 scale.
-template <int W>
-NA_DEVICE void w_load(const WSrc& s, int rblk, int t, int lane, uint4& c, uint32_t& sc) {
-  const int q = lane >> 4, n = lane & 15;
-  const int r = rblk * 16 + n;
-  const int g = min(4 * t + q, kGK - 1);             // groups 90, 91 of the last k-tile: zeroed at the use
-  c = load16<true>(s.codes + (long long)r * kRowBytes + 16 * g);
-  if constexpr (W == kWRaw) {
-    sc = s.scales[(long long)r * kGK + g];
-  } else {
-    const uint8_t* row = s.scales + (long long)r * kPs4Row;
-    const uint32_t nib = row[1 + (g >> 1)];
-    sc = row[0] + ((g & 1) ? (nib >> 4) : (nib & 15));
-  }
-}
 
 constexpr int kPNB = 3;                  // row blocks per wave in the plain, grouped and down kernels
 constexpr int kPRows = 4 * kPNB * 16;    // 192 weight rows per workgroup
@@ -189,36 +175,40 @@ constexpr int kYPitch = 2 * kPRows + 16;              // LDS bytes per row of a 
 constexpr int kOhPitch = 2 * kPKT + 8;                 // LDS bytes per row of gate_up's staged h codes (rows 4 apart
                                                        // start 8 banks apart)
 
-// Staging of one k-tile of 64 q rows: pieces of 16 B, thread tid owns piece (tid & 15) of rows (tid >> 4) + 16 i
-// (pieces 0..7 hi, 8..15 lo); threads 0..63 also own the 4 hi and 4 lo scale bytes of row tid, stored interleaved
-// (hi g, lo g) per group g of the k-tile.
+// Staging of one k-tile of the 16 NT q rows that a tile's tokens fill: pieces of 16 B, thread tid owns piece (tid & 15)
+// of rows (tid >> 4) + 16 i, i < NT (pieces 0..7 hi, 8..15 lo); threads 0..16 NT - 1 also own the 4 hi and 4 lo scale
+// bytes of row tid, stored interleaved (hi g, lo g) per group g of the k-tile.
+template <int NT>
 struct QStage {
-  uint4 v[4];
+  uint4 v[NT];
   uint2 s;
 };
 
 // Activation rows that arrive quantised (q rows): rp[i] = q row of staged row (tid >> 4) + 16 i, srow = q row of
 // staged row tid & 63.
 struct QRows {
-  using Stage = QStage;
+  template <int NT>
+  using Stage = QStage<NT>;
   const uint8_t* rp[4];
   const uint8_t* srow;
 
-  NA_DEVICE void load(int t, int tid, QStage& a) const {
+  template <int NT>
+  NA_DEVICE void load(int t, int tid, QStage<NT>& a) const {
     const int c16 = tid & 15, e0 = t * kPKT + 16 * (c16 & 7), half = (c16 >> 3) * kQLo;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < NT; ++i)
       a.v[i] = e0 < kH ? *reinterpret_cast<const uint4*>(rp[i] + half + e0) : make_uint4(0, 0, 0, 0);
-    if (tid < 64) {
+    if (tid < 16 * NT) {
       a.s.x = *reinterpret_cast<const uint32_t*>(srow + kQSh + 4 * t);
       a.s.y = *reinterpret_cast<const uint32_t*>(srow + kQSl + 4 * t);
     }
   }
-  NA_DEVICE void store(uint8_t* buf, int tid, const QStage& a) const {
+  template <int NT>
+  NA_DEVICE void store(uint8_t* buf, int tid, const QStage<NT>& a) const {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < NT; ++i)
       *reinterpret_cast<uint4*>(buf + ((tid >> 4) + 16 * i) * kQPitch + 16 * (tid & 15)) = a.v[i];
-    if (tid < 64)                                      // interleaved at the store, so the loads are not waited on early
+    if (tid < 16 * NT)                                 // interleaved at the store, so the loads are not waited on early
       *reinterpret_cast<uint2*>(buf + kPBM * kQPitch + 8 * tid) =
           make_uint2(__byte_perm(a.s.x, a.s.y, 0x5140), __byte_perm(a.s.x, a.s.y, 0x7362));
   }
@@ -227,24 +217,28 @@ struct QRows {
 // bf16 activation rows quantised while they are staged (the GEMM entry points, which have no workspace): thread tid
 // owns the 8-element piece tid & 15 of rows (tid >> 4) + 16 i, so the 4 pieces of a 32-element block sit in 4
 // consecutive lanes, as x8_quant_chunk needs.  rp[i] = bf16 row of staged row (tid >> 4) + 16 i.
+template <int NT>
 struct XStage {
-  uint4 v[4];
+  uint4 v[NT];
 };
 
 struct XRows {
-  using Stage = XStage;
+  template <int NT>
+  using Stage = XStage<NT>;
   const uint16_t* rp[4];
 
-  NA_DEVICE void load(int t, int tid, XStage& a) const {
+  template <int NT>
+  NA_DEVICE void load(int t, int tid, XStage<NT>& a) const {
     const int e0 = t * kPKT + 8 * (tid & 15);
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < NT; ++i)
       a.v[i] = e0 < kH ? *reinterpret_cast<const uint4*>(rp[i] + e0) : make_uint4(0, 0, 0, 0);
   }
-  NA_DEVICE void store(uint8_t* buf, int tid, const XStage& a) const {
+  template <int NT>
+  NA_DEVICE void store(uint8_t* buf, int tid, const XStage<NT>& a) const {
     const int c16 = tid & 15;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
+    for (int i = 0; i < NT; ++i) {
       uint2 hi, lo;
       uint32_t sh, sl;
       x8_quant_chunk(a.v[i], hi, lo, sh, sl);
@@ -264,50 +258,83 @@ NA_DEVICE mfma_i32x8_t w_operand8(uint4 c, int t, int lane) {
   return mfma_i32x8_t{(int)c.x, (int)c.y, (int)c.z, (int)c.w, 0, 0, 0, 0};
 }
 
-constexpr int kWScBytes = kTRows * kTScalePitch;      // 1,536 E8M0 bytes of one t950 row block
+constexpr int kWScBytes = kTRows * kTScalePitch;      // LDS bytes of one row block's staged scale rows (t950: 1,536)
 
-// One wave's weight stream over its NB row blocks.  t950: the code bytes of a k-tile per load (the E8M0 rows of the
-// blocks are staged once in the wave's LDS area wsc and read per k-tile from there); raw / PS4: codes and the lane's
-// scale per load.
+// Store layouts: the scale rows of a row block are contiguous (16 x 90 or 16 x 46 bytes), so they are staged as they
+// stand: a k-tile's scale is one LDS byte (PS4: a nibble of one, plus the row's base, which stays in a register).
+// Scattered per-k-tile byte loads in their place (one or two per row block, each 16 lines) bound these layouts before.
+template <int W>
+struct WScales {
+  static constexpr int kPitch = W == kWT950 ? kTScalePitch : W == kWRaw ? kGK : kPs4Row;
+  static constexpr int kBytes = kTRows * kPitch;       // a multiple of 16 in every layout
+  static_assert(kBytes <= kWScBytes && kBytes % 16 == 0, "scale rows of a row block");
+};
+
+// One wave's weight stream over its NB row blocks: the code bytes of a k-tile, one 16-byte load per lane and row block
+// in the MFMA's operand order, at 32-bit offsets from the matrix (lane (q, n): t950 the 16 bytes at 1024 t + 16 lane of
+// the block, raw / PS4 those of group 4t + q of row n; groups 90, 91 re-read group 89 and are zeroed at the use).  The
+// E8M0 rows of the blocks are staged once in the wave's LDS area wsc (stage_scales) and read per k-tile from there.
 template <int W, int NB>
 struct WStream {
   WSrc src;
   const int* blk;
-  const uint8_t* wsc;
+  uint8_t* wsc;
   int lane;
+  int base[NB];                                        // PS4: base byte of this lane's row, per row block
 
-  NA_DEVICE void load(int t, uint4 (&c)[NB], uint32_t (&sc)[NB]) const {
+  NA_DEVICE void load(int t, uint4 (&c)[NB]) const {
+    const int g = min(4 * t + (lane >> 4), kGK - 1);
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
-      if constexpr (W == kWT950) {
-        const uint8_t* bk = src.codes + (long long)blk[nb] * kTBlock;
-        c[nb] = load16(bk + t * 1024 + 16 * lane);
-        sc[nb] = 0;
-      } else {
-        w_load<W>(src, blk[nb], t, lane, c[nb], sc[nb]);
-      }
+      if constexpr (W == kWT950)
+        c[nb] = load16(src.codes + (long long)blk[nb] * kTBlock + t * 1024 + 16 * lane);
+      else
+        c[nb] = load16(src.codes + (uint32_t)((blk[nb] * 16 + (lane & 15)) * kRowBytes + 16 * g));
     }
   }
-  NA_DEVICE int scale(int t, int nb, uint32_t sc) const {
-    if constexpr (W == kWT950)
-      return wsc[nb * kWScBytes + (lane & 15) * kTScalePitch + 4 * t + (lane >> 4)];
-    else
-      return (int)(sc & 0xff);
+  // The blocks' scale rows to LDS, by 16-byte pieces (a view of byte-aligned scales, which only the GEMM entry points
+  // accept: byte by byte).
+  NA_DEVICE void stage_scales() {
+    constexpr int kBytes = WScales<W>::kBytes;
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      const uint8_t* sp = W == kWT950 ? src.codes + (long long)blk[nb] * kTBlock + kTCodes
+                                      : src.scales + (long long)blk[nb] * kBytes;
+      uint8_t* dst = wsc + nb * kWScBytes;
+      if (W == kWT950 || (reinterpret_cast<uintptr_t>(sp) & 15) == 0) {
+#pragma unroll
+        for (int p0 = 0; p0 < kBytes / 16; p0 += 64)
+          if (p0 + lane < kBytes / 16) *reinterpret_cast<uint4*>(dst + 16 * (p0 + lane)) = load16(sp + 16 * (p0 + lane));
+      } else {
+        for (int i = lane; i < kBytes; i += 64) dst[i] = sp[i];
+      }
+      if constexpr (W == kWPs4) base[nb] = sp[(lane & 15) * kPs4Row];
+    }
+  }
+  NA_DEVICE int scale(int t, int nb) const {
+    const uint8_t* row = wsc + nb * kWScBytes + (lane & 15) * WScales<W>::kPitch;
+    const int kb = lane >> 4;
+    if constexpr (W == kWT950) {
+      return row[4 * t + kb];
+    } else if constexpr (W == kWRaw) {
+      return row[min(4 * t + kb, kGK - 1)];
+    } else {
+      return base[nb] + ((row[1 + min(2 * t + (kb >> 1), kGK / 2 - 1)] >> (4 * (kb & 1))) & 15);
+    }
   }
 };
 
-// One k-tile of gemm8_tile.  A of k-tile t is staged in LDS at cur and the weights of k-tile t are in (c, sc).  It
-// issues the loads of A of k-tile t + 2 (into a_in) and of the weights of k-tile t + 2 (into (c2, sc2)), runs the
+// One k-tile of gemm8_tile.  A of k-tile t is staged in LDS at cur and the weights of k-tile t are in c.  It
+// issues the loads of A of k-tile t + 2 (into a_in) and of the weights of k-tile t + 2 (into c2), runs the
 // MFMAs, stores A of k-tile t + 1 (loaded one step earlier, a_out) at nxt and meets the barrier.
 template <int W, int NB, int NT, typename S>
 NA_DEVICE void gemm8_step(int t, const WStream<W, NB>& ws, bool live, const S& st, const uint8_t* cur, uint8_t* nxt,
-                          const typename S::Stage& a_out, typename S::Stage& a_in,
-                          const uint4 (&c)[NB], const uint32_t (&sc)[NB], uint4 (&c2)[NB], uint32_t (&sc2)[NB],
-                          f32x4_t (&acc)[4][NB]) {
+                          const typename S::template Stage<NT>& a_out, typename S::template Stage<NT>& a_in,
+                          const uint4 (&c)[NB], uint4 (&c2)[NB], f32x4_t (&acc)[4][NB]) {
   const int tid = threadIdx.x, lane = tid & 63, kb = lane >> 4, m = lane & 15;
   if (t + 2 < kPTiles) {
-    st.load(t + 2, tid, a_in);
-    ws.load(t + 2, c2, sc2);
+    st.template load<NT>(t + 2, tid, a_in);
+    ws.load(t + 2, c2);
   }
   if (live) {
     mfma_i32x8_t b[NB];
@@ -315,7 +342,7 @@ NA_DEVICE void gemm8_step(int t, const WStream<W, NB>& ws, bool live, const S& s
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) {
       b[nb] = w_operand8(c[nb], t, lane);
-      sb[nb] = ws.scale(t, nb, sc[nb]);
+      sb[nb] = ws.scale(t, nb);
     }
     __builtin_amdgcn_s_setprio(1);                     // the MFMA burst issues ahead of the other wave's staging
 #pragma unroll
@@ -337,11 +364,11 @@ NA_DEVICE void gemm8_step(int t, const WStream<W, NB>& ws, bool live, const S& s
   // The MFMAs are issued before the LDS stores, which wait for their k-tile's loads: an empty asm that takes every
   // accumulator (and orders memory) keeps the compiler from sinking the MFMAs below those stores.
 #pragma unroll
-  for (int tt = 0; tt < 4; ++tt)
+  for (int tt = 0; tt < NT; ++tt)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) asm volatile("" : "+v"(acc[tt][nb])::"memory");
   __builtin_amdgcn_s_setprio(0);
-  if (t + 1 < kPTiles) st.store(nxt, tid, a_out);
+  if (t + 1 < kPTiles) st.template store<NT>(nxt, tid, a_out);
   __syncthreads();
 }
 
@@ -352,8 +379,8 @@ NA_DEVICE void gemm8_step(int t, const WStream<W, NB>& ws, bool live, const S& s
 // 256 code bytes and 8 scale bytes each, loaded into registers two steps before and stored one step before their
 // use), each wave's weight codes through three register sets; the k-loop is unrolled by 3 so that every buffer and
 // register set is fixed at compile time.  Each wave reads one token tile's hi and lo fragments at a time and feeds
-// them to its NB row blocks.  lds: 3 x kQStage bytes; wsc: this wave's LDS area of NB x 1,536 bytes (t950 scale
-// rows).  A wave without work (live = false) stages and meets every barrier but runs no MFMA.  All 256 threads must
+// them to its NB row blocks.  lds: 3 x kQStage bytes; wsc: this wave's LDS area of NB x 1,536 bytes (staged
+// scale rows).  A wave without work (live = false) stages and meets every barrier but runs no MFMA.  All 256 threads must
 // call it.
 template <int W, int NB, int NT, typename S>
 NA_DEVICE void gemm8_tile_n(const WSrc& src, const int (&blk)[NB], bool live, const S& st, uint8_t* lds, uint8_t* wsc,
@@ -363,48 +390,38 @@ NA_DEVICE void gemm8_tile_n(const WSrc& src, const int (&blk)[NB], bool live, co
   for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[tt][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const WStream<W, NB> ws{src, blk, wsc, lane};
-  if constexpr (W == kWT950) {                         // the blocks' E8M0 rows: 96 pieces of 16 B each
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      const uint8_t* sp = src.codes + (long long)blk[nb] * kTBlock + kTCodes;
-      const uint4 v0 = load16(sp + 16 * lane);
-      *reinterpret_cast<uint4*>(wsc + nb * kWScBytes + 16 * lane) = v0;
-      if (lane < kWScBytes / 16 - 64) {
-        const uint4 v1 = load16(sp + 1024 + 16 * lane);
-        *reinterpret_cast<uint4*>(wsc + nb * kWScBytes + 1024 + 16 * lane) = v1;
-      }
-    }
-  }
+  WStream<W, NB> ws{src, blk, wsc, lane, {}};
+  ws.stage_scales();
   uint8_t* const b0 = lds;
   uint8_t* const b1 = lds + kQStage;
   uint8_t* const b2 = lds + 2 * kQStage;
   uint4 c0[NB], c1[NB], c2[NB];
-  uint32_t s0[NB], s1[NB], s2[NB];
-  typename S::Stage a0, a1, a2;                        // a_k: A of the k-tiles = k (mod 3) while in flight
-  st.load(0, tid, a0);
-  ws.load(0, c0, s0);
-  st.load(1, tid, a1);
-  ws.load(1, c1, s1);
-  st.store(b0, tid, a0);
+  typename S::template Stage<NT> a0, a1, a2;           // a_k: A of the k-tiles = k (mod 3) while in flight
+  st.template load<NT>(0, tid, a0);
+  ws.load(0, c0);
+  st.template load<NT>(1, tid, a1);
+  ws.load(1, c1);
+  st.template store<NT>(b0, tid, a0);
   __syncthreads();
   int t = 0;
   for (; t + 3 <= kPTiles; t += 3) {                   // k-tiles 0 .. 20
-    gemm8_step<W, NB, NT, S>(t, ws, live, st, b0, b1, a1, a2, c0, s0, c2, s2, acc);
-    gemm8_step<W, NB, NT, S>(t + 1, ws, live, st, b1, b2, a2, a0, c1, s1, c0, s0, acc);
-    gemm8_step<W, NB, NT, S>(t + 2, ws, live, st, b2, b0, a0, a1, c2, s2, c1, s1, acc);
+    gemm8_step<W, NB, NT, S>(t, ws, live, st, b0, b1, a1, a2, c0, c2, acc);
+    gemm8_step<W, NB, NT, S>(t + 1, ws, live, st, b1, b2, a2, a0, c1, c0, acc);
+    gemm8_step<W, NB, NT, S>(t + 2, ws, live, st, b2, b0, a0, a1, c2, c1, acc);
   }
-  gemm8_step<W, NB, NT, S>(t, ws, live, st, b0, b1, a1, a2, c0, s0, c2, s2, acc);       // 21
-  gemm8_step<W, NB, NT, S>(t + 1, ws, live, st, b1, b2, a2, a0, c1, s1, c0, s0, acc);   // 22
+  gemm8_step<W, NB, NT, S>(t, ws, live, st, b0, b1, a1, a2, c0, c2, acc);       // 21
+  gemm8_step<W, NB, NT, S>(t + 1, ws, live, st, b1, b2, a2, a0, c1, c0, acc);   // 22
 }
 
-// gemm8_tile_n for a tile whose rows fill ntt (1..4) 16-token blocks: the MFMAs of empty blocks are not issued
-// (variants for 1, 2 and 4 blocks; 3 runs as 4).  ntt is workgroup-uniform.
+// gemm8_tile_n for a tile whose rows fill ntt (1..4) 16-token blocks: empty blocks are neither staged nor multiplied.
+// ntt is workgroup-uniform.
 template <int W, int NB, typename S>
 NA_DEVICE void gemm8_tile(const WSrc& src, const int (&blk)[NB], bool live, int ntt, const S& st, uint8_t* lds,
                           uint8_t* wsc, f32x4_t (&acc)[4][NB]) {
-  if (ntt > 2)
+  if (ntt > 3)
     gemm8_tile_n<W, NB, 4, S>(src, blk, live, st, lds, wsc, acc);
+  else if (ntt == 3)
+    gemm8_tile_n<W, NB, 3, S>(src, blk, live, st, lds, wsc, acc);
   else if (ntt == 2)
     gemm8_tile_n<W, NB, 2, S>(src, blk, live, st, lds, wsc, acc);
   else
@@ -429,7 +446,7 @@ NA_DEVICE void xcd_tile(int b, int& tile, int& col) {
 // (one wave's columns of one row) with its own E8M0 scales.  Grid: max tiles x 24 (xcd_tile<3>); in column group 22
 // waves 2 and 3 have no blocks.
 template <int W>
-__global__ __launch_bounds__(256, W == kWT950 ? 2 : 1) void k_prefill_gate_up(
+__global__ __launch_bounds__(256, 2) void k_prefill_gate_up(
     const uint8_t* __restrict__ xq, const int* __restrict__ order, const PTile* __restrict__ tiles,
     const int* __restrict__ ntiles, const uint8_t* __restrict__ pool, long long slot_bytes,
     const int64_t* __restrict__ slot_tab, long long expert_base, const uint16_t* __restrict__ bias_gu,
@@ -542,7 +559,7 @@ __global__ __launch_bounds__(256, W == kWT950 ? 2 : 1) void k_prefill_gate_up(
 // pair of sorted position p0 + m.  A = the h q rows of the tile (consecutive sorted positions).  Grid: max tiles x 16
 // (xcd_tile<2>); wave w: row blocks 12 y + 3 w + i.
 template <int W>
-__global__ __launch_bounds__(256, W == kWT950 ? 2 : 1) void k_prefill_down(
+__global__ __launch_bounds__(256, 2) void k_prefill_down(
     const uint8_t* __restrict__ hq, const int* __restrict__ order, const PTile* __restrict__ tiles,
     const int* __restrict__ ntiles, const uint16_t* __restrict__ wts, const uint8_t* __restrict__ pool,
     long long slot_bytes, const int64_t* __restrict__ slot_tab, long long expert_base,
@@ -607,7 +624,8 @@ __global__ __launch_bounds__(256, W == kWT950 ? 2 : 1) void k_prefill_down(
 }
 
 // ------------------------------------------------------------------------------- plain GEMM (mxfp4_gemm)
-// out[e][m][n] = bf16(sum_k x[m][k] w_e[n][k]); grid (E * ceil(M / 64), N / 192); wave w: row blocks 12 y + 3 w + i.
+// out[e][m][n] = bf16(sum_k x[m][k] w_e[n][k]); tiles = E * ceil(M / 64) of 64 rows; column group y, wave w: row
+// blocks 12 y + 3 w + i.
 // The same block-scaled tiles as the fused layer, the activations quantised into hi + lo rows while staged.
 NA_DEVICE void store_tile(uint16_t* out_row0, long long pitch, const f32x4_t (&acc)[4][kPNB], const int (&blk)[kPNB],
                           int m_limit) {
@@ -626,56 +644,80 @@ NA_DEVICE void store_tile(uint16_t* out_row0, long long pitch, const f32x4_t (&a
       }
 }
 
+// Workgroup of the GEMM entry points -> (tile, column group of 192 rows), a linear grid.  slots > 0: xcd_tile's order
+// with `slots` column groups per XCD, so that each weight row stays in one XCD's L2 while the tiles of its expert pass;
+// slots = 0 (few column groups, which would leave XCDs idle): column groups of a tile in turn.
+NA_DEVICE void gemm_tile_col(int b, int slots, int cols, int& tile, int& col) {
+  if (slots > 0) {
+    const int s = b >> 3;
+    tile = s / slots;
+    col = slots * (b & 7) + (s - tile * slots);
+  } else {
+    tile = b / cols;
+    col = b - tile * cols;
+  }
+}
+
 template <int W>
 __global__ __launch_bounds__(256, 2) void k_mxfp4_gemm(const uint16_t* __restrict__ x, int M,
                                                        const uint8_t* __restrict__ blocks, long long sb_slot,
                                                        const uint8_t* __restrict__ scales, long long ss_slot,
                                                        const int64_t* __restrict__ slots, uint16_t* __restrict__ out,
-                                                       int N) {
+                                                       int N, int xcd_slots) {
   __shared__ __align__(16) uint8_t lds[3 * kQStage + 4 * kPNB * kWScBytes];
   const int mt = (M + kPBM - 1) / kPBM;
-  const int e = blockIdx.x / mt, m0 = (blockIdx.x - e * mt) * kPBM;
+  int i, y;
+  gemm_tile_col(blockIdx.x, xcd_slots, N / kPRows, i, y);
+  if (y >= N / kPRows) return;
+  const int e = i / mt, m0 = (i - e * mt) * kPBM;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int blk[kPNB];
 #pragma unroll
-  for (int i = 0; i < kPNB; ++i) blk[i] = blockIdx.y * (4 * kPNB) + kPNB * wave + i;
+  for (int i = 0; i < kPNB; ++i) blk[i] = y * (4 * kPNB) + kPNB * wave + i;
   const WSrc src = w_src<W>(blocks, sb_slot, scales, ss_slot, slots[e]);
   XRows st;
 #pragma unroll
   for (int i = 0; i < 4; ++i) st.rp[i] = x + (long long)min(m0 + (tid >> 4) + 16 * i, M - 1) * kH;
   f32x4_t acc[4][kPNB];
-  gemm8_tile_n<W, kPNB, 4>(src, blk, true, st, lds, lds + 3 * kQStage + wave * kPNB * kWScBytes, acc);
+  const int ntt = (min(M - m0, kPBM) + 15) >> 4;
+  gemm8_tile<W, kPNB>(src, blk, true, ntt, st, lds, lds + 3 * kQStage + wave * kPNB * kWScBytes, acc);
   store_tile(out + ((long long)e * M + m0) * N, N, acc, blk, M - m0);
 }
 
 // --------------------------------------------------------------- grouped GEMM (GroupedGemmPlan descriptors)
 // tiles int64 [ntiles][5] = (x address, out address, slot, pair M, pm); rows [pm * block_m, min(M, pm * block_m +
-// block_m)) of the pair, walked in 64-row sub-tiles (block_m <= 64: one).  grid (ntiles, N / 192).
+// block_m)) of the pair, as sub-tiles of 64 rows (block_m <= 64: one).
 template <int W>
-__global__ __launch_bounds__(256) void k_mxfp4_gemm_grouped(const uint8_t* __restrict__ blocks, long long sb_slot,
+__global__ __launch_bounds__(256, 2) void k_mxfp4_gemm_grouped(const uint8_t* __restrict__ blocks, long long sb_slot,
                                                                const uint8_t* __restrict__ scales, long long ss_slot,
-                                                               const int64_t* __restrict__ tiles, int block_m, int N) {
+                                                               const int64_t* __restrict__ tiles, int block_m, int N,
+                                                               int xcd_slots) {
   __shared__ __align__(16) uint8_t lds[3 * kQStage + 4 * kPNB * kWScBytes];
-  const int64_t* d = tiles + (long long)blockIdx.x * 5;
+  const int sub = max(block_m / kPBM, 1);              // 64-row sub-tiles per tile, one workgroup each
+  int i, y;
+  gemm_tile_col(blockIdx.x, xcd_slots, N / kPRows, i, y);
+  if (y >= N / kPRows) return;
+  const int64_t* d = tiles + (long long)(i / sub) * 5;
   const uint16_t* x = reinterpret_cast<const uint16_t*>(d[0]);
   uint16_t* out = reinterpret_cast<uint16_t*>(d[1]);
   const long long slot = d[2];
   const int M = (int)d[3], pm = (int)d[4];
+  const long long row0 = (long long)pm * block_m + (i % sub) * kPBM;
+  const int r1 = (int)min((long long)M, (pm + 1LL) * block_m);
+  if (row0 >= r1) return;
+  const int m0 = (int)row0;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   int blk[kPNB];
 #pragma unroll
-  for (int i = 0; i < kPNB; ++i) blk[i] = blockIdx.y * (4 * kPNB) + kPNB * wave + i;
+  for (int i = 0; i < kPNB; ++i) blk[i] = y * (4 * kPNB) + kPNB * wave + i;
   const WSrc src = w_src<W>(blocks, sb_slot, scales, ss_slot, slot);
-  const int r0 = pm * block_m, r1 = min(M, r0 + block_m);
-  for (int m0 = r0; m0 < r1; m0 += kPBM) {
-    XRows st;
+  XRows st;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) st.rp[i] = x + (long long)min(m0 + (tid >> 4) + 16 * i, r1 - 1) * kH;
-    f32x4_t acc[4][kPNB];
-    gemm8_tile_n<W, kPNB, 4>(src, blk, true, st, lds, lds + 3 * kQStage + wave * kPNB * kWScBytes, acc);
-    store_tile(out + (long long)m0 * N, N, acc, blk, r1 - m0);
-    __syncthreads();                                   // the next sub-tile restages the scale rows and buffers
-  }
+  for (int i = 0; i < 4; ++i) st.rp[i] = x + (long long)min(m0 + (tid >> 4) + 16 * i, r1 - 1) * kH;
+  f32x4_t acc[4][kPNB];
+  const int ntt = (min(r1 - m0, kPBM) + 15) >> 4;
+  gemm8_tile<W, kPNB>(src, blk, true, ntt, st, lds, lds + 3 * kQStage + wave * kPNB * kWScBytes, acc);
+  store_tile(out + (long long)m0 * N, N, acc, blk, r1 - m0);
 }
 
 // out[t][n] = bf16(sum_k ys[4 t + k][n]) over the valid ranks k, fp32 sum in top-k order (server.py:2340-2341).
@@ -733,6 +775,14 @@ static PrefillWs prefill_ws(int T) {
   w.ys = align256(w.h + P * kQRow);
   w.total = align256(w.ys + P * kH * 2);
   return w;
+}
+
+// Grid of the GEMM entry points over `tiles` x N / 192 column groups (gemm_tile_col): the XCD order where its 8 x slots
+// column groups are at least 7/8 in use (N = 5760: 30 of 32, N = 2880: 15 of 16), else the plain order.
+static long long gemm_grid(long long tiles, int N, int& xcd_slots) {
+  const int cols = N / kPRows, slots = (cols + 7) / 8;
+  xcd_slots = 8 * cols >= 7 * 8 * slots ? slots : 0;
+  return tiles * (xcd_slots ? 8 * slots : cols);
 }
 
 template <typename... KArgs, typename... Args>
@@ -821,10 +871,13 @@ int na_mxfp4_gemm(const void* x, int M, int K, const void* blocks, long long sb_
   if ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(out)) & 15) return kErrArgs;
   const long long mt = (M + kPBM - 1) / kPBM;
   if (mt * E > 0x7fffffff) return kErrTooLarge;
-  const dim3 grid((unsigned)(mt * E), N / kPRows), blk(256);
+  int xcd_slots;
+  const long long wgs = gemm_grid(mt * E, N, xcd_slots);
+  if (wgs > 0x7fffffff) return kErrTooLarge;
+  const dim3 grid((unsigned)wgs), blk(256);
   auto kern = layout == kWT950 ? k_mxfp4_gemm<kWT950> : layout == kWPs4 ? k_mxfp4_gemm<kWPs4> : k_mxfp4_gemm<kWRaw>;
   hipLaunchKernelGGL(kern, grid, blk, 0, stream, (const uint16_t*)x, M, (const uint8_t*)blocks, sb_slot,
-                     (const uint8_t*)scales, ss_slot, slots, (uint16_t*)out, N);
+                     (const uint8_t*)scales, ss_slot, slots, (uint16_t*)out, N, xcd_slots);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 
@@ -834,11 +887,14 @@ int na_mxfp4_gemm_grouped(const void* blocks, long long sb_slot, const void* sca
   if (K != kH || N % kPRows || layout < kWRaw || layout > kWT950 || (layout != kWT950 && !scales)) return kErrArgs;
   if (block_m < 16 || (block_m & (block_m - 1)) || block_m > 4096) return kErrArgs;
   if (ntiles == 0) return kOk;
-  const dim3 grid(ntiles, N / kPRows), blk(256);
+  int xcd_slots;
+  const long long wgs = gemm_grid((long long)ntiles * max(block_m / kPBM, 1), N, xcd_slots);
+  if (wgs > 0x7fffffff) return kErrTooLarge;
+  const dim3 grid((unsigned)wgs), blk(256);
   auto kern = layout == kWT950 ? k_mxfp4_gemm_grouped<kWT950>
             : layout == kWPs4 ? k_mxfp4_gemm_grouped<kWPs4> : k_mxfp4_gemm_grouped<kWRaw>;
   hipLaunchKernelGGL(kern, grid, blk, 0, stream, (const uint8_t*)blocks, sb_slot, (const uint8_t*)scales, ss_slot,
-                     tiles, block_m, N);
+                     tiles, block_m, N, xcd_slots);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 

@@ -1,0 +1,79 @@
+"""The GEMM entry points at the edges of their tiles: 1 to 4 16-row blocks per tile (full and one row over), column
+counts on both sides of the XCD order's rule (192 and 384 columns take the plain order, 1,536, 2,880 and 5,760 the XCD
+order), scale views that are not 16-byte aligned, and grouped tiles of more than 64 rows.
+
+Bar, per element: one bf16 rounding (8 significant bits: half a unit in the last place is at most 2^-8 of the value,
+reached just above a power of two) of the exact product and fp32 accumulation of the hi and lo rows'
+5,760 products (5,760 x 2^-24 of the sum of their magnitudes); the inputs are N(0, 1), whose products the hi + lo rows
+hold exactly up to 2^-21 of a block's largest magnitude, below the accumulation term."""
+import numpy as np
+import pytest
+
+from oracle import mxfp4_oracle as mo
+from neural_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def slots():
+    rng = np.random.default_rng(91)
+    raw = [synth.slot_raw(rng) for _ in range(2)]
+    return raw, [mo.expert_weights(s)[0].astype(np.float64) for s in raw]
+
+
+def _views(slots, packed, n, odd):
+    """gate_up views of the first n rows; odd: the scale rows copied to an odd address."""
+    import torch
+    from neural_amd.moe.layout import GPTOSS_LAYOUT, GPTOSS_LAYOUT_PS4, mxfp4_pool_views
+    pool = torch.from_numpy(np.stack([mo.ps4_pack_slot(s) if packed else s for s in slots[0]])).cuda()
+    gb, _, gs, _ = mxfp4_pool_views(pool, GPTOSS_LAYOUT_PS4 if packed else GPTOSS_LAYOUT)
+    gb, gs = gb[:, :n], gs[:, :n]
+    if odd:
+        buf = torch.empty(gs.numel() + 1, dtype=torch.uint8, device="cuda")
+        own = buf[1:].view(gs.shape)
+        own.copy_(gs)
+        gs = own
+    return gb, gs
+
+
+def _check(got, x, w, tag):
+    want = x @ w.T
+    bound = 2.0 ** -8 * np.abs(want) + 5760 * 2.0 ** -24 * (np.abs(x) @ np.abs(w).T) + 1e-30
+    worst = (np.abs(got - want) / bound).max(initial=0.0)
+    assert worst <= 1.0, (tag, worst)
+
+
+@pytest.mark.parametrize("n,packed,odd", [(5760, False, False), (2880, True, False), (1536, False, True),
+                                          (384, True, True), (192, False, False)])
+def test_gemm_tile_edges(slots, n, packed, odd):
+    import torch
+    from neural_amd.q80 import mxfp4_kernels as mk
+    gb, gs = _views(slots, packed, n, odd)
+    sl = torch.tensor([1, 0], dtype=torch.int64, device="cuda")
+    rng = np.random.default_rng(n)
+    for M in (1, 16, 17, 32, 33, 48, 49, 65):
+        print(f"case gemm n={n} packed={packed} odd={odd} M={M}", flush=True)
+        x = synth.bf16_normal(rng, (M, 2880))
+        got = mk.mxfp4_gemm(x.cuda(), gb, gs, sl).float().cpu().numpy().astype(np.float64)
+        xf = x.float().numpy().astype(np.float64)
+        for e, s in enumerate((1, 0)):
+            _check(got[e], xf, slots[1][s][:n], (n, packed, odd, M, e))
+
+
+@pytest.mark.parametrize("block_m", [16, 32, 256])
+def test_grouped_sub_tiles(slots, block_m):
+    import torch
+    from neural_amd.q80 import mxfp4_kernels as mk
+    n = 2880
+    gb, gs = _views(slots, False, n, False)
+    rng = np.random.default_rng(block_m)
+    ms = [300, 1, 40, 0, 256, 257]
+    xs = [synth.bf16_normal(rng, (m, 2880)) for m in ms]
+    outs = [torch.full((m, n), 7.0, dtype=torch.bfloat16, device="cuda") for m in ms]
+    print(f"case grouped block_m={block_m} M={ms}", flush=True)
+    mk.mxfp4_gemm_grouped_into([(x.cuda(), i % 2, o) for i, (x, o) in enumerate(zip(xs, outs))], gb, gs,
+                               block_m=block_m)
+    for i, (x, o) in enumerate(zip(xs, outs)):
+        _check(o.float().cpu().numpy().astype(np.float64), x.float().numpy().astype(np.float64),
+               slots[1][i % 2][:n], (block_m, i))
