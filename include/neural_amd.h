@@ -78,6 +78,11 @@ int na_router_topk(const void* xn, int B, const void* w_router, const void* b_ro
  * against an integer round-to-nearest-even: n floats in, three uint16 [n] outputs (hardware, hardware pair, integer). */
 int na_selftest_bf16(const float* in, void* out_hw, void* out_pk, void* out_int, long long n, hipStream_t stream);
 
+/* Device self-check of the clamped SwiGLU the expert kernels use: n (even) bf16 gate and up values in, two bf16 [n]
+ * outputs (the single and the paired form). */
+int na_selftest_swiglu(const void* g, const void* u, float alpha, float limit, void* out, void* out2, long long n,
+                       hipStream_t stream);
+
 /* Device self-check of the MFMA operand layout the tile kernels use: d [16, 16] fp32 = a [16, 32] x b [32, 16] bf16. */
 int na_selftest_mfma(const void* a, const void* b, float* d, hipStream_t stream);
 

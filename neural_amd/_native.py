@@ -26,6 +26,7 @@ SIGNATURES = {
     "na_router_topk": [VP, I32, VP, VP, I32, VP, VP, VP, VP, VP],
     "na_selftest_mfma": [VP, VP, VP, VP],
     "na_selftest_bf16": [VP, VP, VP, VP, I64, VP],
+    "na_selftest_swiglu": [VP, VP, F32, F32, VP, VP, I64, VP],
     "na_selftest_x8": [VP, I32, VP, VP, VP, VP],
     "na_selftest_mfma8": [VP, VP, VP, VP, VP, VP],
     "na_bench_mfma_rate": [I32, I32, I32, VP, VP, VP],

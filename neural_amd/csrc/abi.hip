@@ -51,6 +51,19 @@ __global__ void k_selftest_bf16(const float* __restrict__ in, uint16_t* __restri
   }
 }
 
+// out[i] = swiglu_clamp_bf16 of (g[i], u[i]) as bf16 bits, out2[i] = the paired form's value, for n (even) pairs.
+__global__ void k_selftest_swiglu(const uint16_t* __restrict__ g, const uint16_t* __restrict__ u, float alpha,
+                                  float limit, uint16_t* __restrict__ out, uint16_t* __restrict__ out2, long long n) {
+  const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  const long long p = i & ~1ll;
+  const float gv[2] = {bf16_to_f32(g[p]), bf16_to_f32(g[p + 1])}, uv[2] = {bf16_to_f32(u[p]), bf16_to_f32(u[p + 1])};
+  float h[2];
+  swiglu_clamp_bf16_2(gv, uv, alpha, limit, h);
+  out[i] = f32_to_bf16(swiglu_clamp_bf16(gv[i & 1], uv[i & 1], alpha, limit));
+  out2[i] = f32_to_bf16(h[i & 1]);
+}
+
 // One row of 2880 bf16 per workgroup (384 threads: chunk c = thread, threads past 360 quantise zeros) through the
 // decode kernels' activation quantiser: hi[r][i], lo[r][i] = the E4M3 codes of element i, sc[r][0][b], sc[r][1][b] =
 // the E8M0 bytes of block b for hi and lo.
@@ -153,6 +166,17 @@ int na_selftest_bf16(const float* in, void* out_hw, void* out_pk, void* out_int,
   if (blocks > 0x7fffffffll) return na::kErrTooLarge;
   hipLaunchKernelGGL(na::k_selftest_bf16, dim3((unsigned)blocks), dim3(256), 0, stream, in, (uint16_t*)out_hw,
                      (uint16_t*)out_pk, (uint16_t*)out_int, n);
+  return hipGetLastError() == hipSuccess ? na::kOk : na::kErrLaunch;
+}
+
+// Activation self-check: n (even) pairs of bf16 gate and up values -> two bf16 [n] arrays (single and paired form).
+int na_selftest_swiglu(const void* g, const void* u, float alpha, float limit, void* out, void* out2, long long n,
+                       hipStream_t stream) {
+  if (!g || !u || !out || !out2 || n <= 0 || (n & 1)) return na::kErrArgs;
+  const long long blocks = (n + 255) / 256;
+  if (blocks > 0x7fffffffll) return na::kErrTooLarge;
+  hipLaunchKernelGGL(na::k_selftest_swiglu, dim3((unsigned)blocks), dim3(256), 0, stream, (const uint16_t*)g,
+                     (const uint16_t*)u, alpha, limit, (uint16_t*)out, (uint16_t*)out2, n);
   return hipGetLastError() == hipSuccess ? na::kOk : na::kErrLaunch;
 }
 

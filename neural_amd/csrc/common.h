@@ -87,6 +87,13 @@ NA_DEVICE uint16_t f32_to_bf16(float f) { return __builtin_bit_cast(uint16_t, (_
 
 NA_DEVICE float rb(float f) { return bf16_to_f32(f32_to_bf16(f)); }
 
+// rb of two values: one conversion for both.
+NA_DEVICE void rb2(float& a, float& b) {
+  const uint32_t p = pack_bf16x2(a, b);
+  a = __uint_as_float(p << 16);
+  b = __uint_as_float(p & 0xffff0000u);
+}
+
 // Two E2M1 codes of byte `sel` of `word` -> packed bf16 pair (low nibble -> element 0 in the low half).
 template <int SEL>
 NA_DEVICE uint32_t fp4x2_to_bf16x2(uint32_t word) {
@@ -180,6 +187,17 @@ NA_DEVICE float row16_max(float v) {
   return fmaxf(v, dpp<0x128>(v));
 }
 
+// Largest of unsigned values (the bit patterns of magnitudes, say) over the 4 lanes of a quad, or the 16 lanes of a row
+// of the wavefront, returned to all of them.  0 is the identity of the unsigned maximum, so each step is one
+// v_max_u32 with a DPP operand (a float maximum takes five: a cleared register, the move, its wait, a canonicalising
+// maximum and the maximum).  Must run with all lanes active.
+template <int CTRL>
+NA_DEVICE uint32_t dpp_umax(uint32_t v) {
+  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, false));
+}
+NA_DEVICE uint32_t quad_umax(uint32_t v) { return dpp_umax<0x4E>(dpp_umax<0xB1>(v)); }
+NA_DEVICE uint32_t row16_umax(uint32_t v) { return dpp_umax<0x128>(dpp_umax<0x124>(quad_umax(v))); }
+
 // Sum over the 64 lanes of a wavefront, returned (wave-uniform) to every lane.  Must run with all lanes active.
 // Fixed order: lane pairs, quads (DPP quad_perm), rows of 16 (DPP row_ror 4, 8), then the four row sums.
 NA_DEVICE float wave_total(float v) {
@@ -194,15 +212,45 @@ NA_DEVICE float wave_total(float v) {
   return (r0 + r1) + (r2 + r3);
 }
 
+// bf16(1 / (1 + exp(-t))) of a bf16 value t, on the hardware's base-2 exponential and reciprocal (both within 1 fp32
+// ulp): the bits of the correctly rounded fp32 expression at every bf16 t except the three (-87.5, -88, -88.5) whose
+// sigmoid is below 2^-126 and becomes +0 (na_selftest_swiglu, all 65,536 arguments).  expf and the IEEE division took
+// about 25 instructions more per value; the epilogue of a full prompt tile (32 values per lane) was 18 % of it.
+NA_DEVICE float sigmoid_bf16(float t) {
+  return rb(__builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t * -1.44269504f)));
+}
+
 // Clamped SwiGLU of one (gate, up) element pair with torch's bf16 op-by-op rounding
-// (reference neural/q80/expert_runtime.py:63-72, server.py:2014-2021): inputs are bf16 values.
+// (reference neural/q80/expert_runtime.py:63-72, server.py:2014-2021): inputs are bf16 values, the result is one.
+// med3(u, -limit, limit) is min(max(u, -limit), limit), NaN included.
 NA_DEVICE float swiglu_clamp_bf16(float g, float u, float alpha, float limit) {
   const float gate = fminf(g, limit);
-  const float up = fminf(fmaxf(u, -limit), limit);
-  const float t = rb(gate * alpha);
-  const float s = rb(1.0f / (1.0f + expf(-t)));
+  const float up = __builtin_amdgcn_fmed3f(u, -limit, limit);
+  const float s = sigmoid_bf16(rb(gate * alpha));
   const float glu = rb(gate * s);
   return rb(rb(up + 1.0f) * glu);
+}
+
+// swiglu_clamp_bf16 of two pairs, the bf16 conversions shared.
+NA_DEVICE void swiglu_clamp_bf16_2(const float (&g)[2], const float (&u)[2], float alpha, float limit, float (&h)[2]) {
+  float gate[2], t[2], s[2], up[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    gate[i] = fminf(g[i], limit);
+    up[i] = __builtin_amdgcn_fmed3f(u[i], -limit, limit) + 1.0f;
+    t[i] = gate[i] * alpha;
+  }
+  rb2(t[0], t[1]);
+  rb2(up[0], up[1]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) s[i] = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t[i] * -1.44269504f));
+  rb2(s[0], s[1]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) s[i] *= gate[i];
+  rb2(s[0], s[1]);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) h[i] = up[i] * s[i];
+  rb2(h[0], h[1]);
 }
 
 }  // namespace na

@@ -58,12 +58,10 @@ NA_DEVICE void x8_quant_chunk(uint4 v, uint2& hi, uint2& lo, uint32_t& sh, uint3
     f[2 * i] = bf16_to_f32((uint16_t)(w[i] & 0xffff));
     f[2 * i + 1] = bf16_to_f32((uint16_t)(w[i] >> 16));
   }
-  float m = 0.f;
+  uint32_t m = 0;                                      // the block's largest magnitude, as bf16 bits
 #pragma unroll
-  for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(f[i]));
-  m = fmaxf(m, __shfl_xor(m, 1));
-  m = fmaxf(m, __shfl_xor(m, 2));
-  sh = x8_scale_byte(m);
+  for (int i = 0; i < 4; ++i) m = max(m, max(w[i] & 0x7fffu, (w[i] >> 16) & 0x7fffu));
+  sh = x8_scale_byte(__uint_as_float(quad_umax(m) << 16));
   const float s_hi = e8m0_f32(sh);
   uint32_t hc[2];
   float r[8];
@@ -83,9 +81,7 @@ NA_DEVICE void x8_quant_chunk(uint4 v, uint2& hi, uint2& lo, uint32_t& sh, uint3
   float mr = 0.f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) mr = fmaxf(mr, fabsf(r[i]));
-  mr = fmaxf(mr, __shfl_xor(mr, 1));
-  mr = fmaxf(mr, __shfl_xor(mr, 2));
-  sl = x8_scale_byte(mr);
+  sl = x8_scale_byte(__uint_as_float(quad_umax(__float_as_uint(mr))));
   const float s_lo = e8m0_f32(sl);
   uint32_t lc[2];
 #pragma unroll
