@@ -308,6 +308,12 @@ int na_core_route_pack(const void* hn, const float* logits, const int64_t* ids, 
                        const int64_t* slot_tab, long long base, void* bx, float* pack, int near_miss, int64_t* bslots,
                        int64_t* bgids, void* bw, hipStream_t stream);
 
+/* na_core_router and na_core_route_pack in one launch, with their arguments and results. */
+int na_core_router_pack(const void* mid, const void* post_w, float eps, const void* Wr, const void* br, void* hn,
+                        float* logits, unsigned int* counter, int64_t* ids, void* wts, const int64_t* slot_tab,
+                        long long base, void* bx, float* pack, int near_miss, int64_t* bslots, int64_t* bgids, void* bw,
+                        hipStream_t stream);
+
 /* The attention block of one decode layer in ONE launch: na_core_qkv, na_decode_attention (B = 1), na_core_oproj and
  * na_core_router, with their arguments and results (fused_core.py:581-629: k_qkv, k_attn / SplitAttn, k_oproj,
  * k_router + k_topk), as four phases of one grid.  Each phase issues its loads (weights; the cache rows of earlier

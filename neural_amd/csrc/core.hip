@@ -365,13 +365,66 @@ __global__ __launch_bounds__(256) void k_oproj(const uint16_t* __restrict__ att,
 // itself): each workgroup counts itself into *entered once its read of the generation word is complete, and the
 // last workgroup, once its own logits are stored, waits for all NR counts (the other phases' workgroups have read
 // the word, since their results fed its mid), returns the count to zero and advances the word.
+// The serving outputs that na_core_router_pack adds to the router's (k_route_pack states them).
+struct RoutePack {
+  const int64_t* slot_tab;
+  long long base;
+  uint16_t* bx;
+  float* pack;
+  int64_t* bslots;
+  int64_t* bgids;
+  uint16_t* bw;
+  int near_miss;
+};
+
+// Rank `lane` (0..3) of the top 4: expert e with weight w.
+NA_DEVICE void route_pack_entries(const RoutePack& rp, int lane, int64_t e, uint16_t w) {
+  const long long g = rp.base + e;
+  const int64_t s = rp.slot_tab ? rp.slot_tab[g] : g;
+  const bool hit = s >= 0;
+  rp.bslots[lane] = hit ? s : 0;
+  rp.bgids[lane] = g;
+  rp.bw[lane] = hit ? w : (uint16_t)0;
+  if (rp.pack) {
+    rp.pack[kH + lane] = bf16_to_f32(w);
+    rp.pack[kH + 4 + lane] = (float)e;
+    rp.pack[kH + 8 + lane] = hit ? 1.f : 0.f;
+  }
+}
+
+// Ranks 5..8: v0, v1 = the logits of experts lane and lane + 64, -inf for the top 4's.  One wave, all lanes.
+NA_DEVICE void route_pack_near(const RoutePack& rp, int lane, float v0, float v1) {
+  for (int r = 0; r < 4; ++r) {
+    float v = v0;
+    int i = lane;
+    if (v1 > v) {                                   // ties keep the lower index
+      v = v1;
+      i = lane + 64;
+    }
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+      const float ov = __shfl_xor(v, o);
+      const int oi = __shfl_xor(i, o);
+      if (ov > v || (ov == v && oi < i)) {
+        v = ov;
+        i = oi;
+      }
+    }
+    if (lane == 0) rp.pack[kH + 12 + r] = (float)i;
+    if (i == lane) v0 = -INFINITY;
+    if (i == lane + 64) v1 = -INFINITY;
+  }
+}
+
+// rp (not FUSED): the serving outputs, written where their inputs already are: workgroup 0's normed mid, the last
+// workgroup's top 4.
 template <int TPR, bool FUSED>
 NA_DEVICE void router_body(int blk, int nr, uint16_t* hc, uint32_t& last, const uint16_t* __restrict__ mid,
                            const uint16_t* __restrict__ post_w, float eps, const uint16_t* __restrict__ Wr,
                            const uint16_t* __restrict__ br, uint16_t* __restrict__ hn, float* __restrict__ logits,
                            uint32_t* __restrict__ counter, int64_t* __restrict__ ids, uint16_t* __restrict__ wts,
                            const uint64_t* mid_tags, uint64_t* logit_tags, uint32_t* gen_word, uint32_t gen,
-                           uint32_t* err, uint32_t* entered = nullptr) {
+                           uint32_t* err, uint32_t* entered = nullptr, const RoutePack* rp = nullptr) {
   constexpr int ROWS = 256 / TPR;
   const int tid = threadIdx.x, r = tid / TPR, j = tid % TPR;
   const int e = ROWS * blk + r;
@@ -409,6 +462,19 @@ NA_DEVICE void router_body(int blk, int nr, uint16_t* hc, uint32_t& last, const 
   if (blk == 0)
     for (int i = tid; i < kH / 8; i += 256)
       *reinterpret_cast<uint4*>(hn + 8 * i) = *reinterpret_cast<const uint4*>(hc + 8 * i);
+  if (!FUSED && rp && blk == 0) {
+    for (int i = tid; i < kH / 2; i += 256) {
+      const uint32_t h2 = *reinterpret_cast<const uint32_t*>(hc + 2 * i);
+      if (rp->bx) {
+        rp->bx[2 * i] = (uint16_t)h2;
+        rp->bx[2 * i + 1] = (uint16_t)(h2 >> 16);
+      }
+      if (rp->pack) {
+        rp->pack[2 * i] = __uint_as_float(h2 << 16);
+        rp->pack[2 * i + 1] = __uint_as_float(h2 & 0xffff0000u);
+      }
+    }
+  }
   const float s = rw.dot(hc, j);
   if constexpr (FUSED) {
     const float v = rb(s + bf16_to_f32(bv));
@@ -447,8 +513,32 @@ NA_DEVICE void router_body(int blk, int nr, uint16_t* hc, uint32_t& last, const 
   }
   __syncthreads();
   if (!last || tid >= 64) return;
-  top4_softmax(__hip_atomic_load(logits + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT),
-               __hip_atomic_load(logits + tid + 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), tid, ids, wts);
+  float v0 = __hip_atomic_load(logits + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  float v1 = __hip_atomic_load(logits + tid + 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if constexpr (!FUSED) {
+    if (rp) {
+      float tv[4];
+      int ti[4];
+      top4_select(v0, v1, tid, tv, ti);
+      if (tid < 4) {
+        const int e4 = top4_id(ti, tid);
+        const uint16_t w4 = top4_weight(tv, tid);
+        ids[tid] = e4;
+        wts[tid] = w4;
+        route_pack_entries(*rp, tid, e4, w4);
+      }
+      if (rp->near_miss) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          if (ti[k] == tid) v0 = -INFINITY;
+          if (ti[k] == tid + 64) v1 = -INFINITY;
+        }
+        route_pack_near(*rp, tid, v0, v1);
+      }
+      return;
+    }
+  }
+  top4_softmax(v0, v1, tid, ids, wts);
 }
 
 template <int TPR>
@@ -461,6 +551,20 @@ __global__ __launch_bounds__(256) void k_router_norm(const uint16_t* __restrict_
   __shared__ uint32_t last;
   router_body<TPR, false>(blockIdx.x, gridDim.x, hc, last, mid, post_w, eps, Wr, br, hn, logits, counter, ids, wts,
                           nullptr, nullptr, nullptr, 0, nullptr);
+}
+
+// The router and its serving outputs in one launch (the drop-in core's last kernel of a layer): as two launches the
+// second, one workgroup that re-reads hn and the top 4, took 6.7 us of a 38 us layer beside its launch.
+template <int TPR>
+__global__ __launch_bounds__(256) void k_router_pack(const uint16_t* __restrict__ mid, const uint16_t* __restrict__ post_w,
+                                                     float eps, const uint16_t* __restrict__ Wr,
+                                                     const uint16_t* __restrict__ br, uint16_t* __restrict__ hn,
+                                                     float* __restrict__ logits, uint32_t* __restrict__ counter,
+                                                     int64_t* __restrict__ ids, uint16_t* __restrict__ wts, RoutePack rp) {
+  __shared__ __align__(16) uint16_t hc[kH];
+  __shared__ uint32_t last;
+  router_body<TPR, false>(blockIdx.x, gridDim.x, hc, last, mid, post_w, eps, Wr, br, hn, logits, counter, ids, wts,
+                          nullptr, nullptr, nullptr, 0, nullptr, nullptr, &rp);
 }
 
 // Monotone map of bf16 bit patterns to unsigned order (-0 equal to +0; NaN patterns above +inf).
@@ -763,20 +867,8 @@ __global__ __launch_bounds__(256) void k_route_pack(const uint16_t* __restrict__
     if (bx) bx[i] = h;
     if (pack) pack[i] = bf16_to_f32(h);
   }
-  if (tid < 4) {
-    const int64_t e = ids[tid];
-    const long long g = base + e;
-    const int64_t s = slot_tab ? slot_tab[g] : g;
-    const bool hit = s >= 0;
-    bslots[tid] = hit ? s : 0;
-    bgids[tid] = g;
-    bw[tid] = hit ? wts[tid] : (uint16_t)0;
-    if (pack) {
-      pack[kH + tid] = bf16_to_f32(wts[tid]);
-      pack[kH + 4 + tid] = (float)e;
-      pack[kH + 8 + tid] = hit ? 1.f : 0.f;
-    }
-  }
+  const RoutePack rp{slot_tab, base, bx, pack, bslots, bgids, bw, near_miss};
+  if (tid < 4) route_pack_entries(rp, tid, ids[tid], wts[tid]);
   if (!near_miss || tid >= 64) return;
   float v0 = logits[tid], v1 = logits[tid + 64];
   for (int j = 0; j < 4; ++j) {
@@ -784,28 +876,8 @@ __global__ __launch_bounds__(256) void k_route_pack(const uint16_t* __restrict__
     if (e == tid) v0 = -INFINITY;
     if (e == tid + 64) v1 = -INFINITY;
   }
-  for (int r = 0; r < 4; ++r) {
-    float v = v0;
-    int i = tid;
-    if (v1 > v) {                                   // ties keep the lower index
-      v = v1;
-      i = tid + 64;
-    }
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      const float ov = __shfl_xor(v, o);
-      const int oi = __shfl_xor(i, o);
-      if (ov > v || (ov == v && oi < i)) {
-        v = ov;
-        i = oi;
-      }
-    }
-    if (tid == 0) pack[kH + 12 + r] = (float)i;
-    if (i == tid) v0 = -INFINITY;
-    if (i == tid + 64) v1 = -INFINITY;
-  }
+  route_pack_near(rp, tid, v0, v1);
 }
-
 
 // ---------------------------------------------------------------- the attention block of a decode layer, one launch
 // Phases by workgroup id (see handoff.h): [QKV: 640][attention: 8 ns][o_proj: 360][router: 32].  Each phase issues
@@ -946,6 +1018,19 @@ int na_core_route_pack(const void* hn, const float* logits, const int64_t* ids, 
   hipLaunchKernelGGL(k_route_pack, dim3(1), dim3(256), 0, stream, (const uint16_t*)hn, logits, ids,
                      (const uint16_t*)wts, slot_tab, base, (uint16_t*)bx, pack, bslots, bgids, (uint16_t*)bw,
                      near_miss ? 1 : 0);
+  return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
+}
+
+int na_core_router_pack(const void* mid, const void* post_w, float eps, const void* Wr, const void* br, void* hn,
+                        float* logits, unsigned int* counter, int64_t* ids, void* wts, const int64_t* slot_tab,
+                        long long base, void* bx, float* pack, int near_miss, int64_t* bslots, int64_t* bgids, void* bw,
+                        hipStream_t stream) {
+  if (!mid || !post_w || !Wr || !br || !hn || !logits || !counter || !ids || !wts) return kErrArgs;
+  if (!bslots || !bgids || !bw || base < 0 || (near_miss && !pack)) return kErrArgs;
+  const RoutePack rp{slot_tab, base, (uint16_t*)bx, pack, bslots, bgids, (uint16_t*)bw, near_miss ? 1 : 0};
+  hipLaunchKernelGGL(k_router_pack<kRouterTpr>, dim3(kNE / (256 / kRouterTpr)), dim3(256), 0, stream,
+                     (const uint16_t*)mid, (const uint16_t*)post_w, eps, (const uint16_t*)Wr, (const uint16_t*)br,
+                     (uint16_t*)hn, logits, (uint32_t*)counter, ids, (uint16_t*)wts, rp);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 

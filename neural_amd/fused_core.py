@@ -19,10 +19,10 @@ and ``k``, ``v``, ``sliding``, ``smax``, ``scaling``, ``h_norm``, ``r_scores``, 
 device), ``inv_freq`` (fp32 [32]) and ``att_scale``.  ``core_graphs(weights, smax, dev)`` builds such an object from a
 neural_amd.model.DecodeWeights, for callers without the reference's eager core.
 
-Per layer, run() is five launches on the current stream (no host synchronisation, nothing read on the host, so it
+Per layer, run() is four launches on the current stream (no host synchronisation, nothing read on the host, so it
 can be captured): na_core_qkv (residual combine + RMSNorm + Q|K|V + bias + RoPE + K/V write), na_decode_attention,
-na_core_oproj, na_core_router (post RMSNorm + router + top-4 + softmax), na_core_route_pack (bx, pack, bslots, bgids,
-bw: the expert body's inputs and the host pack).
+na_core_oproj, na_core_router_pack (post RMSNorm + router + top-4 + softmax, and bx, pack, bslots, bgids, bw: the
+expert body's inputs and the host pack).
 """
 from __future__ import annotations
 
@@ -182,10 +182,9 @@ class FusedCore:
         N.call("na_core_oproj", self.att.data_ptr(), a.o_proj.weight.data_ptr(), a.o_proj.bias.data_ptr(),
                self.xbuf.data_ptr(), mid.data_ptr(), s)
         r = ly.mlp.router
-        N.call("na_core_router", mid.data_ptr(), ly.post_attention_layernorm.weight.data_ptr(),
+        N.call("na_core_router_pack", mid.data_ptr(), ly.post_attention_layernorm.weight.data_ptr(),
                float(ly.post_attention_layernorm.variance_epsilon), r.weight.data_ptr(), r.bias.data_ptr(),
-               hn_o.data_ptr(), self.logits.data_ptr(), self.counter.data_ptr(), idx_o.data_ptr(), sc_o.data_ptr(), s)
-        N.call("na_core_route_pack", hn_o.data_ptr(), self.logits.data_ptr(), idx_o.data_ptr(), sc_o.data_ptr(),
+               hn_o.data_ptr(), self.logits.data_ptr(), self.counter.data_ptr(), idx_o.data_ptr(), sc_o.data_ptr(),
                N.ptr(slot_tab), L * NE, bx.data_ptr(), pack.data_ptr(), int(self.near_miss), bslots.data_ptr(),
                bgids.data_ptr(), bw.data_ptr(), s)
 
