@@ -11,11 +11,13 @@
 // so an output deviates from the reference's by at most 2^-21 sum_k |w_k| m_k before its bf16 rounding (t950.h
 // states the quantiser).
 //
-// The plain and grouped GEMM entry points (bf16 activations, no workspace) run the same tiles, the activations
-// quantised into hi + lo rows while they are staged.  They are HBM-bound where experts have few rows: 2,000 Zipf-routed
-// rows over a raw store, gate_up and down, 1,390 -> 536 us (1.7 GB; bit-identical) when the scales went through LDS
-// instead of scattered byte loads, tiles stopped staging and multiplying their empty 16-row blocks, column groups got
-// the XCD order, and the kernels, 400 registers before, came to fit two workgroups per CU.
+// The plain and grouped GEMM entry points (bf16 activations, no workspace) run the same tiles on bf16 rows and
+// v_mfma_f32_16x16x32_bf16, the weights converted to bf16 (exact) in registers.  They are HBM-bound where experts have
+// few rows: 2,000 Zipf-routed rows over a raw store, gate_up and down, 1,390 -> 493 us (1.7 GB) when the scales went
+// through LDS instead of scattered byte loads, tiles stopped staging and multiplying their empty 16-row blocks, column
+// groups got the XCD order, and the kernels, 400 registers before, came to fit two workgroups per CU; 493 -> 462 us,
+// and one expert's 4,096 rows 320 -> 213 us (957 TFLOP/s), when the rows stopped being quantised into hi + lo E4M3
+// rows by every column group.
 //
 // Weight layouts (template W): the store's raw and PS4 slots (row r: 1,440 code bytes, then a raw 90-byte or PS4
 // 46-byte scale row; lane (q, n) reads the 16 bytes of group 4t + q of row n, already the MFMA's B order) and the t950
@@ -38,6 +40,13 @@ struct WSrc {
   const uint8_t* codes;     // raw/PS4: row 0's code bytes (row pitch 1,440); t950: block 0 of the matrix
   const uint8_t* scales;    // raw/PS4: row 0's scale row (pitch 90 or 46); t950: unused
 };
+
+// Two E2M1 codes of byte SEL of `word`, times 2^e of the float `scale` -> packed bf16 pair (low nibble = element 0 in the
+// low half): exact for every E8M0 scale byte of 1 .. 254.
+template <int SEL>
+NA_DEVICE uint32_t fp4x2_scaled(uint32_t word, float scale) {
+  return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, scale, SEL));
+}
 
 constexpr int kPNB = 3;                  // row blocks per wave in the plain, grouped and down kernels
 constexpr int kPRows = 4 * kPNB * 16;    // 192 weight rows per workgroup
@@ -187,6 +196,7 @@ struct QStage {
 // Activation rows that arrive quantised (q rows): rp[i] = q row of staged row (tid >> 4) + 16 i, srow = q row of
 // staged row tid & 63.
 struct QRows {
+  static constexpr bool kBf16 = false;
   template <int NT>
   using Stage = QStage<NT>;
   const uint8_t* rp[4];
@@ -214,40 +224,31 @@ struct QRows {
   }
 };
 
-// bf16 activation rows quantised while they are staged (the GEMM entry points, which have no workspace): thread tid
-// owns the 8-element piece tid & 15 of rows (tid >> 4) + 16 i, so the 4 pieces of a 32-element block sit in 4
-// consecutive lanes, as x8_quant_chunk needs.  rp[i] = bf16 row of staged row (tid >> 4) + 16 i.
+// bf16 activation rows staged as they are (the GEMM entry points): thread tid owns the 8-element piece tid & 15 of rows
+// (tid >> 4) + 16 i.  rp[i] = bf16 row of staged row (tid >> 4) + 16 i.
 template <int NT>
-struct XStage {
+struct BStage {
   uint4 v[NT];
 };
 
-struct XRows {
+struct BRows {
+  static constexpr bool kBf16 = true;
   template <int NT>
-  using Stage = XStage<NT>;
+  using Stage = BStage<NT>;
   const uint16_t* rp[4];
 
   template <int NT>
-  NA_DEVICE void load(int t, int tid, XStage<NT>& a) const {
+  NA_DEVICE void load(int t, int tid, BStage<NT>& a) const {
     const int e0 = t * kPKT + 8 * (tid & 15);
 #pragma unroll
     for (int i = 0; i < NT; ++i)
       a.v[i] = e0 < kH ? *reinterpret_cast<const uint4*>(rp[i] + e0) : make_uint4(0, 0, 0, 0);
   }
   template <int NT>
-  NA_DEVICE void store(uint8_t* buf, int tid, const XStage<NT>& a) const {
-    const int c16 = tid & 15;
+  NA_DEVICE void store(uint8_t* buf, int tid, const BStage<NT>& a) const {
 #pragma unroll
-    for (int i = 0; i < NT; ++i) {
-      uint2 hi, lo;
-      uint32_t sh, sl;
-      x8_quant_chunk(a.v[i], hi, lo, sh, sl);
-      const int row = (tid >> 4) + 16 * i;
-      *reinterpret_cast<uint2*>(buf + row * kQPitch + 8 * c16) = hi;
-      *reinterpret_cast<uint2*>(buf + row * kQPitch + kPKT + 8 * c16) = lo;
-      if ((c16 & 3) == 0)
-        *reinterpret_cast<uint16_t*>(buf + kPBM * kQPitch + row * 8 + 2 * (c16 >> 2)) = (uint16_t)(sh | (sl << 8));
-    }
+    for (int i = 0; i < NT; ++i)
+      *reinterpret_cast<uint4*>(buf + ((tid >> 4) + 16 * i) * kQPitch + 16 * (tid & 15)) = a.v[i];
   }
 };
 
@@ -340,6 +341,71 @@ struct WStream {
   }
 };
 
+// The MFMAs of k-tile t on quantised rows staged at cur, weight codes c: block-scaled, hi and lo rows.
+template <int W, int NB, int NT>
+NA_DEVICE void ktile_x8(int t, const WStream<W, NB>& ws, const uint8_t* cur, const uint4 (&c)[NB], f32x4_t (&acc)[4][NB]) {
+  const int lane = threadIdx.x & 63, kb = lane >> 4, m = lane & 15;
+  mfma_i32x8_t b[NB];
+  int sb[NB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) {
+    b[nb] = w_operand8(c[nb], t, lane);
+    sb[nb] = ws.scale(t, nb);
+  }
+  __builtin_amdgcn_s_setprio(1);                     // the MFMA burst issues ahead of the other wave's staging
+#pragma unroll
+  for (int tt = 0; tt < NT; ++tt) {
+    const uint8_t* row = cur + (16 * tt + m) * kQPitch + 16 * kb;
+    const uint4 h0 = *reinterpret_cast<const uint4*>(row), h1 = *reinterpret_cast<const uint4*>(row + 64);
+    const uint4 l0 = *reinterpret_cast<const uint4*>(row + 128), l1 = *reinterpret_cast<const uint4*>(row + 192);
+    const uint32_t s2 = *reinterpret_cast<const uint16_t*>(cur + kPBM * kQPitch + (16 * tt + m) * 8 + 2 * kb);
+    const int sh = (int)(s2 & 0xff), sl = (int)(s2 >> 8);
+    const mfma_i32x8_t ah = {(int)h0.x, (int)h0.y, (int)h0.z, (int)h0.w, (int)h1.x, (int)h1.y, (int)h1.z, (int)h1.w};
+    const mfma_i32x8_t al = {(int)l0.x, (int)l0.y, (int)l0.z, (int)l0.w, (int)l1.x, (int)l1.y, (int)l1.z, (int)l1.w};
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      acc[tt][nb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ah, b[nb], acc[tt][nb], 0, 4, 0, sh, 0, sb[nb]);
+      acc[tt][nb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(al, b[nb], acc[tt][nb], 0, 4, 0, sl, 0, sb[nb]);
+    }
+  }
+}
+
+// The MFMAs of k-tile t on bf16 rows: the E2M1 codes x 2^(s - 127) converted to bf16 (exact), 16 conversions per row
+// block and k-tile shared by the tile's 16-token blocks.  v_mfma_f32_16x16x32_bf16 at half the scaled instruction's
+// rate and one row instead of hi and lo: the same matrix-core time, the reference's exact products, and no
+// quantisation of the rows (which each of the 15 to 30 column groups repeated: about 220 vector instructions per
+// k-tile of a full tile against the 48 conversions).  MFMA j multiplies elements 8 j .. 8 j + 7 of each of the k-tile's
+// four 32-element groups (lane 16 kb + m: group kb), on both operands.
+template <int W, int NB, int NT>
+NA_DEVICE void ktile_bf16(int t, const WStream<W, NB>& ws, const uint8_t* cur, const uint4 (&c)[NB],
+                          f32x4_t (&acc)[4][NB]) {
+  const int lane = threadIdx.x & 63, kb = lane >> 4, m = lane & 15;
+  uint4 b[NB][4];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) {
+    const bool in = 4 * t + kb < kGK;
+    const uint32_t w[4] = {in ? c[nb].x : 0u, in ? c[nb].y : 0u, in ? c[nb].z : 0u, in ? c[nb].w : 0u};
+    const float s = e8m0_f32((uint32_t)ws.scale(t, nb) & 0xff);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      b[nb][j] = make_uint4(fp4x2_scaled<0>(w[j], s), fp4x2_scaled<1>(w[j], s), fp4x2_scaled<2>(w[j], s),
+                            fp4x2_scaled<3>(w[j], s));
+  }
+  __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+  for (int tt = 0; tt < NT; ++tt) {
+    const uint8_t* row = cur + (16 * tt + m) * kQPitch + 64 * kb;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const bf16x8_t a = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(row + 16 * j));
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb)
+        acc[tt][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, __builtin_bit_cast(bf16x8_t, b[nb][j]), acc[tt][nb],
+                                                              0, 0, 0);
+    }
+  }
+}
+
 // One k-tile of gemm8_tile.  A of k-tile t is staged in LDS at cur and the weights of k-tile t are in c.  It
 // issues the loads of A of k-tile t + 2 (into a_in) and of the weights of k-tile t + 2 (into c2), runs the
 // MFMAs, stores A of k-tile t + 1 (loaded one step earlier, a_out) at nxt and meets the barrier.
@@ -347,35 +413,14 @@ template <int W, int NB, int NT, typename S>
 NA_DEVICE void gemm8_step(int t, const WStream<W, NB>& ws, bool live, const S& st, const uint8_t* cur, uint8_t* nxt,
                           const typename S::template Stage<NT>& a_out, typename S::template Stage<NT>& a_in,
                           const uint4 (&c)[NB], uint4 (&c2)[NB], f32x4_t (&acc)[4][NB]) {
-  const int tid = threadIdx.x, lane = tid & 63, kb = lane >> 4, m = lane & 15;
+  const int tid = threadIdx.x;
   if (t + 2 < kPTiles) {
     st.template load<NT>(t + 2, tid, a_in);
     ws.load(t + 2, c2);
   }
   if (live) {
-    mfma_i32x8_t b[NB];
-    int sb[NB];
-#pragma unroll
-    for (int nb = 0; nb < NB; ++nb) {
-      b[nb] = w_operand8(c[nb], t, lane);
-      sb[nb] = ws.scale(t, nb);
-    }
-    __builtin_amdgcn_s_setprio(1);                     // the MFMA burst issues ahead of the other wave's staging
-#pragma unroll
-    for (int tt = 0; tt < NT; ++tt) {
-      const uint8_t* row = cur + (16 * tt + m) * kQPitch + 16 * kb;
-      const uint4 h0 = *reinterpret_cast<const uint4*>(row), h1 = *reinterpret_cast<const uint4*>(row + 64);
-      const uint4 l0 = *reinterpret_cast<const uint4*>(row + 128), l1 = *reinterpret_cast<const uint4*>(row + 192);
-      const uint32_t s2 = *reinterpret_cast<const uint16_t*>(cur + kPBM * kQPitch + (16 * tt + m) * 8 + 2 * kb);
-      const int sh = (int)(s2 & 0xff), sl = (int)(s2 >> 8);
-      const mfma_i32x8_t ah = {(int)h0.x, (int)h0.y, (int)h0.z, (int)h0.w, (int)h1.x, (int)h1.y, (int)h1.z, (int)h1.w};
-      const mfma_i32x8_t al = {(int)l0.x, (int)l0.y, (int)l0.z, (int)l0.w, (int)l1.x, (int)l1.y, (int)l1.z, (int)l1.w};
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb) {
-        acc[tt][nb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ah, b[nb], acc[tt][nb], 0, 4, 0, sh, 0, sb[nb]);
-        acc[tt][nb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(al, b[nb], acc[tt][nb], 0, 4, 0, sl, 0, sb[nb]);
-      }
-    }
+    if constexpr (S::kBf16) ktile_bf16<W, NB, NT>(t, ws, cur, c, acc);
+    else ktile_x8<W, NB, NT>(t, ws, cur, c, acc);
   }
   // The MFMAs are issued before the LDS stores, which wait for their k-tile's loads: an empty asm that takes every
   // accumulator (and orders memory) keeps the compiler from sinking the MFMAs below those stores.
@@ -390,7 +435,7 @@ NA_DEVICE void gemm8_step(int t, const WStream<W, NB>& ws, bool live, const S& s
 
 // acc[tt][nb] = D of tokens 16 tt .. 16 tt + 15 x row block blk[nb] (lane (q, n): tokens 16 tt + 4 q + r, row n),
 // over the 23 k-tiles for tt < NT (the 16-token blocks that hold rows; the others stay zero); st stages the
-// activation rows (QRows or XRows).  Both
+// activation rows (QRows or BRows).  Both
 // operand streams run two k-tiles ahead of the MFMAs: the activations through three LDS buffers of a k-tile (64 rows'
 // 256 code bytes and 8 scale bytes each, loaded into registers two steps before and stored one step before their
 // use), each wave's weight codes through three register sets; the k-loop is unrolled by 3 so that every buffer and
@@ -660,7 +705,7 @@ __global__ __launch_bounds__(256, 2) void k_prefill_down(
 // ------------------------------------------------------------------------------- plain GEMM (mxfp4_gemm)
 // out[e][m][n] = bf16(sum_k x[m][k] w_e[n][k]); tiles = E * ceil(M / 64) of 64 rows; column group y, wave w: row
 // blocks 12 y + 3 w + i.
-// The same block-scaled tiles as the fused layer, the activations quantised into hi + lo rows while staged.
+// The fused layer's tiles on bf16 rows (ktile_bf16).
 NA_DEVICE void store_tile(uint16_t* out_row0, long long pitch, const f32x4_t (&acc)[4][kPNB], const int (&blk)[kPNB],
                           int m_limit) {
   const int lane = threadIdx.x & 63, q = lane >> 4, n = lane & 15;
@@ -709,7 +754,7 @@ __global__ __launch_bounds__(256, 2) void k_mxfp4_gemm(const uint16_t* __restric
 #pragma unroll
   for (int i = 0; i < kPNB; ++i) blk[i] = y * (4 * kPNB) + kPNB * wave + i;
   const WSrc src = w_src<W>(blocks, sb_slot, scales, ss_slot, slots[e]);
-  XRows st;
+  BRows st;
 #pragma unroll
   for (int i = 0; i < 4; ++i) st.rp[i] = x + (long long)min(m0 + (tid >> 4) + 16 * i, M - 1) * kH;
   f32x4_t acc[4][kPNB];
@@ -745,7 +790,7 @@ __global__ __launch_bounds__(256, 2) void k_mxfp4_gemm_grouped(const uint8_t* __
 #pragma unroll
   for (int i = 0; i < kPNB; ++i) blk[i] = y * (4 * kPNB) + kPNB * wave + i;
   const WSrc src = w_src<W>(blocks, sb_slot, scales, ss_slot, slot);
-  XRows st;
+  BRows st;
 #pragma unroll
   for (int i = 0; i < 4; ++i) st.rp[i] = x + (long long)min(m0 + (tid >> 4) + 16 * i, r1 - 1) * kH;
   f32x4_t acc[4][kPNB];

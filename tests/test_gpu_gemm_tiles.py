@@ -3,9 +3,8 @@ counts on both sides of the XCD order's rule (192 and 384 columns take the plain
 order), scale views that are not 16-byte aligned, and grouped tiles of more than 64 rows.
 
 Bar, per element: one bf16 rounding (8 significant bits: half a unit in the last place is at most 2^-8 of the value,
-reached just above a power of two) of the exact product and fp32 accumulation of the hi and lo rows'
-5,760 products (5,760 x 2^-24 of the sum of their magnitudes); the inputs are N(0, 1), whose products the hi + lo rows
-hold exactly up to 2^-21 of a block's largest magnitude, below the accumulation term."""
+reached just above a power of two) of the exact product and fp32 accumulation of 2,880 exact
+products (below 5,760 x 2^-24 of the sum of their magnitudes)."""
 import numpy as np
 import pytest
 
