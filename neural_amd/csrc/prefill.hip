@@ -3,17 +3,21 @@
 // each output; reference neural/q80/mxfp4_kernels.py:87-126, 242-295) and the fused MoE prefill layer (reference
 // server.py:1837-1936, _expert_gemms :1977-2040).
 //
-// Every kernel here runs the same tiles (ptile): bf16 activation rows as they are, the weights' E2M1 codes converted to
-// bf16 with their E8M0 scale in registers (exact), v_mfma_f32_16x16x32_bf16.  The block-scaled FP8 x FP4 instruction,
-// which takes the codes as stored, needs the activations as hi + lo E4M3 rows: the same matrix-core time for two rows,
-// and the rows' quantisation (x by a launch's threads, h in the gate_up epilogue, or in the GEMM entry points by every
-// column group).  Measured against it: the MoE layer of 2,048 tokens 630 -> 610 us, 600 tokens 376 -> 362, raw stores
-// 803 -> 703; mxfp4_gemm of 4,096 rows 320 -> 213 (957 TFLOP/s); the error against 64 bits is the same.
+// The fused layer (k_prefill_gate_up / k_prefill_down) runs on the block-scaled v_mfma_scale_f32_16x16x128_f8f6f4:
+// E2M1 codes and E8M0 scales as stored, activations as two E4M3 rows (hi, lo) with one E8M0 scale per 32 elements
+// each (x per 32-element block of a row; h per 32 columns of a row, quantised in the gate_up epilogue).  hi w + lo w
+// is the reference's bf16 x E2M1 product exactly for every element within 2^13 of its block's largest magnitude m;
+// an element further below m is reproduced to within 2^-21 m (the remainder's 4 significant bits on the lo grid),
+// so an output deviates from the reference's by at most 2^-21 sum_k |w_k| m_k before its bf16 rounding (t950.h
+// states the quantiser).
 //
-// Where experts have few rows the products are HBM-bound: 2,000 Zipf-routed rows over a raw store (grouped gate_up and
-// down, 1.7 GB) take 462 us, 1,390 before the scales went through LDS instead of scattered byte loads, tiles stopped
-// staging and multiplying their empty 16-row blocks, column groups got the XCD order and the kernels, 400 registers
-// before, came to fit two workgroups per CU.
+// The plain and grouped GEMM entry points (bf16 activations, no workspace) run the same tiles on bf16 rows and
+// v_mfma_f32_16x16x32_bf16, the weights converted to bf16 (exact) in registers.  They are HBM-bound where experts have
+// few rows: 2,000 Zipf-routed rows over a raw store, gate_up and down, 1,390 -> 493 us (1.7 GB) when the scales went
+// through LDS instead of scattered byte loads, tiles stopped staging and multiplying their empty 16-row blocks, column
+// groups got the XCD order, and the kernels, 400 registers before, came to fit two workgroups per CU; 493 -> 462 us,
+// and one expert's 4,096 rows 320 -> 213 us (957 TFLOP/s), when the rows stopped being quantised into hi + lo E4M3
+// rows by every column group.
 //
 // Weight layouts (template W): the store's raw and PS4 slots (row r: 1,440 code bytes, then a raw 90-byte or PS4
 // 46-byte scale row; lane (q, n) reads the 16 bytes of group 4t + q of row n, already the MFMA's B order) and the t950
@@ -37,8 +41,8 @@ struct WSrc {
   const uint8_t* scales;    // raw/PS4: row 0's scale row (pitch 90 or 46); t950: unused
 };
 
-// Two E2M1 codes of byte SEL of `word`, times 2^e of the float `scale` -> packed bf16 pair (low nibble = element 0 in
-// the low half): exact for every E8M0 scale byte of 1 .. 254.
+// Two E2M1 codes of byte SEL of `word`, times 2^e of the float `scale` -> packed bf16 pair (low nibble = element 0 in the
+// low half): exact for every E8M0 scale byte of 1 .. 254.
 template <int SEL>
 NA_DEVICE uint32_t fp4x2_scaled(uint32_t word, float scale) {
   return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, scale, SEL));
@@ -58,12 +62,45 @@ NA_DEVICE WSrc w_src(const uint8_t* blocks, long long sb_slot, const uint8_t* sc
 // pairs by expert (order[offs[e] + i] = the i-th pair of expert e in increasing p) and a tile table
 // tiles[i] = (expert, first sorted position, rows <= 64), ntiles.  Invalid ids are in no expert's list and
 // contribute +0 (the combine skips them).
+// Quantised row ("q row", kQRow bytes): hi codes [0, 2880), lo codes [2880, 5760), hi scales [5760, 5856) and lo
+// scales [5856, 5952), scale bytes 90..95 of each half zero (the last k-tile's groups 90, 91 are padding).
+constexpr int kQRow = 2 * kH + 2 * kX8ScPitch;        // 5,952
+constexpr int kQLo = kH;
+constexpr int kQSh = 2 * kH;
+constexpr int kQSl = 2 * kH + kX8ScPitch;
+
 struct PTile {
   int e, p0, cnt, pad;
 };
 
-// Block e: counts[e] = pairs routed to expert e.
-__global__ __launch_bounds__(256) void k_prefill_count(const int64_t* __restrict__ ids, int P, int* __restrict__ counts) {
+// Blocks 0..127: counts[e] = pairs routed to expert e.  Blocks 128..: x quantised into q rows, one 8-element chunk
+// per thread (4 consecutive threads = one 32-element block; 360 chunks per row, so a block never straddles rows).
+__global__ __launch_bounds__(256) void k_prefill_count(const int64_t* __restrict__ ids, int P, int* __restrict__ counts,
+                                                       const uint16_t* __restrict__ x, int T, uint8_t* __restrict__ xq) {
+  if (blockIdx.x >= 128) {
+    const long long g = (long long)(blockIdx.x - 128) * 256 + threadIdx.x;
+    const bool ok = g < (long long)T * kChunks;
+    const long long row = ok ? g / kChunks : 0;
+    const int c = ok ? (int)(g - row * kChunks) : 0;
+    const uint4 v = ok ? *reinterpret_cast<const uint4*>(x + row * kH + 8 * c) : make_uint4(0, 0, 0, 0);
+    uint2 hi, lo;
+    uint32_t sh, sl;
+    x8_quant_chunk(v, hi, lo, sh, sl);
+    if (ok) {
+      uint8_t* dst = xq + row * kQRow;
+      *reinterpret_cast<uint2*>(dst + 8 * c) = hi;
+      *reinterpret_cast<uint2*>(dst + kQLo + 8 * c) = lo;
+      if ((c & 3) == 0) {
+        dst[kQSh + (c >> 2)] = (uint8_t)sh;
+        dst[kQSl + (c >> 2)] = (uint8_t)sl;
+      }
+      if (c < kX8ScPitch - kGK) {
+        dst[kQSh + kGK + c] = 0;
+        dst[kQSl + kGK + c] = 0;
+      }
+    }
+    return;
+  }
   const int e = blockIdx.x;
   __shared__ int part[4];
   int c = 0;
@@ -131,13 +168,61 @@ __global__ __launch_bounds__(256) void k_prefill_order(const int64_t* __restrict
   }
 }
 
-// ------------------------------------------------------------------------------------------- prompt tiles
-constexpr int kAPitch = 2 * kPKT + 16;                 // LDS bytes per staged row of a k-tile: 128 bf16 | pad 16
-constexpr int kAStage = kPBM * kAPitch;                // one k-tile of 64 rows
+// ---------------------------------------------------------------- block-scaled products of the fused layer
+// The layer's two GEMMs run on v_mfma_scale_f32_16x16x128_f8f6f4 with the E2M1 codes and E8M0 scales as stored (B)
+// and the activations as two exact E4M3 rows (A: hi and lo, one E8M0 scale per 32-element block each; the exactness
+// argument is the one of x8_quant_chunk in t950.h).  Each k-tile of 128 elements is one MFMA per (16 tokens, 16 weight
+// rows) and activation row (hi, lo): the hi + lo products are the reference's bf16 x E2M1 products, accumulated in
+// fp32.  Activations are quantised once per row, not per workgroup: x per token by the first launch, h per sorted pair
+// by the gate_up epilogue.
+//
+constexpr int kQPitch = 2 * kPKT + 16;                 // LDS bytes per staged row: hi 128 | lo 128 | pad 16
+constexpr int kQStage = kPBM * kQPitch + kPBM * 8;     // one k-tile: 64 rows, then 8 scale bytes per row
 constexpr int kGuSlots = 3;                            // gate_up: 23 column groups over 8 XCDs, 3 per XCD
 constexpr int kDnSlots = 2;                            // down: 15 column groups, 2 per XCD
 constexpr int kYPitch = 2 * kPRows + 16;              // LDS bytes per row of a staged down output tile
-constexpr int kOhPitch = 2 * kPKT + 16;                // LDS bytes per row of gate_up's staged h columns
+constexpr int kOhPitch = 2 * kPKT + 8;                 // LDS bytes per row of gate_up's staged h codes (rows 4 apart
+                                                       // start 8 banks apart)
+
+// Staging of one k-tile of the 16 NT q rows that a tile's tokens fill: pieces of 16 B, thread tid owns piece (tid & 15)
+// of rows (tid >> 4) + 16 i, i < NT (pieces 0..7 hi, 8..15 lo); threads 0..16 NT - 1 also own the 4 hi and 4 lo scale
+// bytes of row tid, stored interleaved (hi g, lo g) per group g of the k-tile.
+template <int NT>
+struct QStage {
+  uint4 v[NT];
+  uint2 s;
+};
+
+// Activation rows that arrive quantised (q rows): rp[i] = q row of staged row (tid >> 4) + 16 i, srow = q row of
+// staged row tid & 63.
+struct QRows {
+  static constexpr bool kBf16 = false;
+  template <int NT>
+  using Stage = QStage<NT>;
+  const uint8_t* rp[4];
+  const uint8_t* srow;
+
+  template <int NT>
+  NA_DEVICE void load(int t, int tid, QStage<NT>& a) const {
+    const int c16 = tid & 15, e0 = t * kPKT + 16 * (c16 & 7), half = (c16 >> 3) * kQLo;
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+      a.v[i] = e0 < kH ? *reinterpret_cast<const uint4*>(rp[i] + half + e0) : make_uint4(0, 0, 0, 0);
+    if (tid < 16 * NT) {
+      a.s.x = *reinterpret_cast<const uint32_t*>(srow + kQSh + 4 * t);
+      a.s.y = *reinterpret_cast<const uint32_t*>(srow + kQSl + 4 * t);
+    }
+  }
+  template <int NT>
+  NA_DEVICE void store(uint8_t* buf, int tid, const QStage<NT>& a) const {
+#pragma unroll
+    for (int i = 0; i < NT; ++i)
+      *reinterpret_cast<uint4*>(buf + ((tid >> 4) + 16 * i) * kQPitch + 16 * (tid & 15)) = a.v[i];
+    if (tid < 16 * NT)                                 // interleaved at the store, so the loads are not waited on early
+      *reinterpret_cast<uint2*>(buf + kPBM * kQPitch + 8 * tid) =
+          make_uint2(__byte_perm(a.s.x, a.s.y, 0x5140), __byte_perm(a.s.x, a.s.y, 0x7362));
+  }
+};
 
 // bf16 activation rows staged as they are (the GEMM entry points): thread tid owns the 8-element piece tid & 15 of rows
 // (tid >> 4) + 16 i.  rp[i] = bf16 row of staged row (tid >> 4) + 16 i.
@@ -147,6 +232,7 @@ struct BStage {
 };
 
 struct BRows {
+  static constexpr bool kBf16 = true;
   template <int NT>
   using Stage = BStage<NT>;
   const uint16_t* rp[4];
@@ -162,9 +248,16 @@ struct BRows {
   NA_DEVICE void store(uint8_t* buf, int tid, const BStage<NT>& a) const {
 #pragma unroll
     for (int i = 0; i < NT; ++i)
-      *reinterpret_cast<uint4*>(buf + ((tid >> 4) + 16 * i) * kAPitch + 16 * (tid & 15)) = a.v[i];
+      *reinterpret_cast<uint4*>(buf + ((tid >> 4) + 16 * i) * kQPitch + 16 * (tid & 15)) = a.v[i];
   }
 };
+
+// FP4 B operand of k-tile t in the MFMA order (lane 16 kb + n: the 16 code bytes of group 4t + kb of row n), groups
+// beyond K zeroed.  Every layout's load already is in that order.
+NA_DEVICE mfma_i32x8_t w_operand8(uint4 c, int t, int lane) {
+  if (4 * t + (lane >> 4) >= kGK) c = make_uint4(0, 0, 0, 0);
+  return mfma_i32x8_t{(int)c.x, (int)c.y, (int)c.z, (int)c.w, 0, 0, 0, 0};
+}
 
 constexpr int kWScBytes = kTRows * kTScalePitch;      // LDS bytes of one row block's staged scale rows (t950: 1,536)
 
@@ -181,8 +274,7 @@ struct WScales {
 // One wave's weight stream over its NB row blocks: the code bytes of a k-tile, one 16-byte load per lane and row block
 // in the MFMA's operand order, at 32-bit offsets from the matrix (lane (q, n): t950 the 16 bytes at 1024 t + 16 lane of
 // the block, raw / PS4 those of group 4t + q of row n; groups 90, 91 re-read group 89 and are zeroed at the use).  The
-// E8M0 rows of the blocks are staged once in the wave's LDS area wsc (load_scales, store_scales) and read per k-tile
-// from there.
+// E8M0 rows of the blocks are staged once in the wave's LDS area wsc (load_scales, store_scales) and read per k-tile from there.
 template <int W, int NB>
 struct WStream {
   WSrc src;
@@ -249,14 +341,43 @@ struct WStream {
   }
 };
 
-// The MFMAs of k-tile t: the E2M1 codes x 2^(s - 127) converted to bf16 (exact), 16 conversions per row
+// The MFMAs of k-tile t on quantised rows staged at cur, weight codes c: block-scaled, hi and lo rows.
+template <int W, int NB, int NT>
+NA_DEVICE void ktile_x8(int t, const WStream<W, NB>& ws, const uint8_t* cur, const uint4 (&c)[NB], f32x4_t (&acc)[4][NB]) {
+  const int lane = threadIdx.x & 63, kb = lane >> 4, m = lane & 15;
+  mfma_i32x8_t b[NB];
+  int sb[NB];
+#pragma unroll
+  for (int nb = 0; nb < NB; ++nb) {
+    b[nb] = w_operand8(c[nb], t, lane);
+    sb[nb] = ws.scale(t, nb);
+  }
+  __builtin_amdgcn_s_setprio(1);                     // the MFMA burst issues ahead of the other wave's staging
+#pragma unroll
+  for (int tt = 0; tt < NT; ++tt) {
+    const uint8_t* row = cur + (16 * tt + m) * kQPitch + 16 * kb;
+    const uint4 h0 = *reinterpret_cast<const uint4*>(row), h1 = *reinterpret_cast<const uint4*>(row + 64);
+    const uint4 l0 = *reinterpret_cast<const uint4*>(row + 128), l1 = *reinterpret_cast<const uint4*>(row + 192);
+    const uint32_t s2 = *reinterpret_cast<const uint16_t*>(cur + kPBM * kQPitch + (16 * tt + m) * 8 + 2 * kb);
+    const int sh = (int)(s2 & 0xff), sl = (int)(s2 >> 8);
+    const mfma_i32x8_t ah = {(int)h0.x, (int)h0.y, (int)h0.z, (int)h0.w, (int)h1.x, (int)h1.y, (int)h1.z, (int)h1.w};
+    const mfma_i32x8_t al = {(int)l0.x, (int)l0.y, (int)l0.z, (int)l0.w, (int)l1.x, (int)l1.y, (int)l1.z, (int)l1.w};
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      acc[tt][nb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(ah, b[nb], acc[tt][nb], 0, 4, 0, sh, 0, sb[nb]);
+      acc[tt][nb] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(al, b[nb], acc[tt][nb], 0, 4, 0, sl, 0, sb[nb]);
+    }
+  }
+}
+
+// The MFMAs of k-tile t on bf16 rows: the E2M1 codes x 2^(s - 127) converted to bf16 (exact), 16 conversions per row
 // block and k-tile shared by the tile's 16-token blocks.  v_mfma_f32_16x16x32_bf16 at half the scaled instruction's
 // rate and one row instead of hi and lo: the same matrix-core time, the reference's exact products, and no
 // quantisation of the rows (which each of the 15 to 30 column groups repeated: about 220 vector instructions per
 // k-tile of a full tile against the 48 conversions).  MFMA j multiplies elements 8 j .. 8 j + 7 of each of the k-tile's
 // four 32-element groups (lane 16 kb + m: group kb), on both operands.
 template <int W, int NB, int NT>
-NA_DEVICE void ptile_mfma(int t, const WStream<W, NB>& ws, const uint8_t* cur, const uint4 (&c)[NB],
+NA_DEVICE void ktile_bf16(int t, const WStream<W, NB>& ws, const uint8_t* cur, const uint4 (&c)[NB],
                           f32x4_t (&acc)[4][NB]) {
   const int lane = threadIdx.x & 63, kb = lane >> 4, m = lane & 15;
   uint4 b[NB][4];
@@ -273,7 +394,7 @@ NA_DEVICE void ptile_mfma(int t, const WStream<W, NB>& ws, const uint8_t* cur, c
   __builtin_amdgcn_s_setprio(1);
 #pragma unroll
   for (int tt = 0; tt < NT; ++tt) {
-    const uint8_t* row = cur + (16 * tt + m) * kAPitch + 64 * kb;
+    const uint8_t* row = cur + (16 * tt + m) * kQPitch + 64 * kb;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const bf16x8_t a = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(row + 16 * j));
@@ -285,11 +406,11 @@ NA_DEVICE void ptile_mfma(int t, const WStream<W, NB>& ws, const uint8_t* cur, c
   }
 }
 
-// One k-tile of ptile.  A of k-tile t is staged in LDS at cur and the weights of k-tile t are in c.  It
+// One k-tile of gemm8_tile.  A of k-tile t is staged in LDS at cur and the weights of k-tile t are in c.  It
 // issues the loads of A of k-tile t + 2 (into a_in) and of the weights of k-tile t + 2 (into c2), runs the
 // MFMAs, stores A of k-tile t + 1 (loaded one step earlier, a_out) at nxt and meets the barrier.
 template <int W, int NB, int NT, typename S>
-NA_DEVICE void ptile_step(int t, const WStream<W, NB>& ws, bool live, const S& st, const uint8_t* cur, uint8_t* nxt,
+NA_DEVICE void gemm8_step(int t, const WStream<W, NB>& ws, bool live, const S& st, const uint8_t* cur, uint8_t* nxt,
                           const typename S::template Stage<NT>& a_out, typename S::template Stage<NT>& a_in,
                           const uint4 (&c)[NB], uint4 (&c2)[NB], f32x4_t (&acc)[4][NB]) {
   const int tid = threadIdx.x;
@@ -298,7 +419,8 @@ NA_DEVICE void ptile_step(int t, const WStream<W, NB>& ws, bool live, const S& s
     ws.load(t + 2, c2);
   }
   if (live) {
-    ptile_mfma<W, NB, NT>(t, ws, cur, c, acc);
+    if constexpr (S::kBf16) ktile_bf16<W, NB, NT>(t, ws, cur, c, acc);
+    else ktile_x8<W, NB, NT>(t, ws, cur, c, acc);
   }
   // The MFMAs are issued before the LDS stores, which wait for their k-tile's loads: an empty asm that takes every
   // accumulator (and orders memory) keeps the compiler from sinking the MFMAs below those stores.
@@ -311,17 +433,18 @@ NA_DEVICE void ptile_step(int t, const WStream<W, NB>& ws, bool live, const S& s
   __syncthreads();
 }
 
-// acc[tt][nb] = D of tokens 16 tt .. 16 tt + 15 x row block blk[nb] (lane (q, n): tokens 16 tt + 4 q + r, row n), over
-// the 23 k-tiles for tt < NT (the 16-token blocks that hold rows; the others stay zero); st stages the activation rows
-// (BRows).  Both operand streams run two k-tiles ahead of the MFMAs: the activations through three LDS buffers of a
-// k-tile (64 rows of 256 bytes, loaded into registers two steps before and stored one step before their use), each
-// wave's weight codes through three register sets; the k-loop is unrolled by 3 so that every buffer and register set is
-// fixed at compile time.  Each wave reads one token tile's fragments at a time and feeds them to its NB row blocks.
-// (Measured, slower: deeper prefetch or two k-tiles per barrier for tiles of one or two 16-row blocks.)  lds: 3 x
-// kAStage bytes; wsc: this wave's LDS area of NB x 1,536 bytes (staged scale rows).  A wave without work (live = false)
-// stages and meets every barrier but runs no MFMA.  All 256 threads must call it.
+// acc[tt][nb] = D of tokens 16 tt .. 16 tt + 15 x row block blk[nb] (lane (q, n): tokens 16 tt + 4 q + r, row n),
+// over the 23 k-tiles for tt < NT (the 16-token blocks that hold rows; the others stay zero); st stages the
+// activation rows (QRows or BRows).  Both
+// operand streams run two k-tiles ahead of the MFMAs: the activations through three LDS buffers of a k-tile (64 rows'
+// 256 code bytes and 8 scale bytes each, loaded into registers two steps before and stored one step before their
+// use), each wave's weight codes through three register sets; the k-loop is unrolled by 3 so that every buffer and
+// register set is fixed at compile time.  Each wave reads one token tile's hi and lo fragments at a time and feeds
+// them to its NB row blocks.  lds: 3 x kQStage bytes; wsc: this wave's LDS area of NB x 1,536 bytes (staged
+// scale rows).  A wave without work (live = false) stages and meets every barrier but runs no MFMA.  All 256 threads must
+// call it.
 template <int W, int NB, int NT, typename S>
-NA_DEVICE void ptile_n(const WSrc& src, const int (&blk)[NB], bool live, const S& st, uint8_t* lds, uint8_t* wsc,
+NA_DEVICE void gemm8_tile_n(const WSrc& src, const int (&blk)[NB], bool live, const S& st, uint8_t* lds, uint8_t* wsc,
                             f32x4_t (&acc)[4][NB]) {
   const int tid = threadIdx.x, lane = tid & 63;
 #pragma unroll
@@ -332,8 +455,8 @@ NA_DEVICE void ptile_n(const WSrc& src, const int (&blk)[NB], bool live, const S
   uint4 wsv[NB][WStream<W, NB>::kScRounds];
   ws.load_scales(wsv);
   uint8_t* const b0 = lds;
-  uint8_t* const b1 = lds + kAStage;
-  uint8_t* const b2 = lds + 2 * kAStage;
+  uint8_t* const b1 = lds + kQStage;
+  uint8_t* const b2 = lds + 2 * kQStage;
   uint4 c0[NB], c1[NB], c2[NB];
   typename S::template Stage<NT> a0, a1, a2;           // a_k: A of the k-tiles = k (mod 3) while in flight
   ws.load(0, c0);
@@ -347,27 +470,27 @@ NA_DEVICE void ptile_n(const WSrc& src, const int (&blk)[NB], bool live, const S
   __syncthreads();
   int t = 0;
   for (; t + 3 <= kPTiles; t += 3) {                   // k-tiles 0 .. 20
-    ptile_step<W, NB, NT, S>(t, ws, live, st, b0, b1, a1, a2, c0, c2, acc);
-    ptile_step<W, NB, NT, S>(t + 1, ws, live, st, b1, b2, a2, a0, c1, c0, acc);
-    ptile_step<W, NB, NT, S>(t + 2, ws, live, st, b2, b0, a0, a1, c2, c1, acc);
+    gemm8_step<W, NB, NT, S>(t, ws, live, st, b0, b1, a1, a2, c0, c2, acc);
+    gemm8_step<W, NB, NT, S>(t + 1, ws, live, st, b1, b2, a2, a0, c1, c0, acc);
+    gemm8_step<W, NB, NT, S>(t + 2, ws, live, st, b2, b0, a0, a1, c2, c1, acc);
   }
-  ptile_step<W, NB, NT, S>(t, ws, live, st, b0, b1, a1, a2, c0, c2, acc);       // 21
-  ptile_step<W, NB, NT, S>(t + 1, ws, live, st, b1, b2, a2, a0, c1, c0, acc);   // 22
+  gemm8_step<W, NB, NT, S>(t, ws, live, st, b0, b1, a1, a2, c0, c2, acc);       // 21
+  gemm8_step<W, NB, NT, S>(t + 1, ws, live, st, b1, b2, a2, a0, c1, c0, acc);   // 22
 }
 
-// ptile_n for a tile whose rows fill ntt (1..4) 16-token blocks: empty blocks are neither staged nor multiplied.
+// gemm8_tile_n for a tile whose rows fill ntt (1..4) 16-token blocks: empty blocks are neither staged nor multiplied.
 // ntt is workgroup-uniform.
 template <int W, int NB, typename S>
-NA_DEVICE void ptile(const WSrc& src, const int (&blk)[NB], bool live, int ntt, const S& st, uint8_t* lds,
+NA_DEVICE void gemm8_tile(const WSrc& src, const int (&blk)[NB], bool live, int ntt, const S& st, uint8_t* lds,
                           uint8_t* wsc, f32x4_t (&acc)[4][NB]) {
   if (ntt > 3)
-    ptile_n<W, NB, 4, S>(src, blk, live, st, lds, wsc, acc);
+    gemm8_tile_n<W, NB, 4, S>(src, blk, live, st, lds, wsc, acc);
   else if (ntt == 3)
-    ptile_n<W, NB, 3, S>(src, blk, live, st, lds, wsc, acc);
+    gemm8_tile_n<W, NB, 3, S>(src, blk, live, st, lds, wsc, acc);
   else if (ntt == 2)
-    ptile_n<W, NB, 2, S>(src, blk, live, st, lds, wsc, acc);
+    gemm8_tile_n<W, NB, 2, S>(src, blk, live, st, lds, wsc, acc);
   else
-    ptile_n<W, NB, 1, S>(src, blk, live, st, lds, wsc, acc);
+    gemm8_tile_n<W, NB, 1, S>(src, blk, live, st, lds, wsc, acc);
 }
 
 // Workgroup b -> (tile, column group): the dispatcher deals workgroups to the 8 XCDs in turn (XCD b % 8), so XCD x
@@ -381,22 +504,24 @@ NA_DEVICE void xcd_tile(int b, int& tile, int& col) {
   col = SLOTS * (b & 7) + s % SLOTS;
 }
 
-// A full tile's workgroup (stamped, cycles, at hi + lo rows): prologue 8,860 -> 5,900 since the weights, their scales
-// and the row addresses are requested side by side; its 23 k-tiles 2,100 each (1,024 of MFMAs; two workgroups share a
-// SIMD); epilogue 15,700 -> 8,700 (32 activations per lane) by the hardware exponential and reciprocal and shared
-// conversions, and less since h leaves as bf16.  Layer: 2,048 tokens 667 -> 610 us, 23 tokens 189 -> 175.
+// A full tile's workgroup (stamped, cycles): prologue 8,860 -> 5,900 since the weights, their scales and the row
+// addresses are requested side by side; its 23 k-tiles 2,100 each (1,024 of MFMAs; two workgroups share a SIMD);
+// epilogue 15,700 -> 8,700 (32 activations per lane) by the hardware exponential and reciprocal, block maxima of one
+// instruction per step and shared conversions.  Layer: 2,048 tokens 665 -> 630 us, 23 tokens 191 -> 182, same bits.
 //
-// gate_up + bias + clamped SwiGLU: tile i, column group y (128 intermediate columns). Wave w owns intermediate blocks
-// jb, jb + 1 (jb = 8 y + 2 w) and reads their gate rows (blocks jb, jb + 1) and up rows (blocks 180 + jb, 181 + jb), so
-// the SwiGLU pairs registers of one lane.  x rows are gathered through the pair order; h leaves as bf16 rows in sorted
-// pair order.  Grid: max tiles x 24 (xcd_tile<3>); in column group 22 waves 2 and 3 have no blocks.
+// gate_up + bias + clamped SwiGLU on the block-scaled MFMA: tile i, column group y (128 intermediate columns).
+// Wave w owns intermediate blocks jb, jb + 1 (jb = 8 y + 2 w) and reads their gate rows (blocks jb, jb + 1) and up
+// rows (blocks 180 + jb, 181 + jb), so the SwiGLU pairs registers of one lane.  x rows come quantised (xq, one q row
+// per token) and are gathered through the pair order; h leaves as q rows in sorted pair order, each 32-column block
+// (one wave's columns of one row) with its own E8M0 scales.  Grid: max tiles x 24 (xcd_tile<3>); in column group 22
+// waves 2 and 3 have no blocks.
 template <int W>
 __global__ __launch_bounds__(256, 2) void k_prefill_gate_up(
-    const uint16_t* __restrict__ x, const int* __restrict__ order, const PTile* __restrict__ tiles,
+    const uint8_t* __restrict__ xq, const int* __restrict__ order, const PTile* __restrict__ tiles,
     const int* __restrict__ ntiles, const uint8_t* __restrict__ pool, long long slot_bytes,
     const int64_t* __restrict__ slot_tab, long long expert_base, const uint16_t* __restrict__ bias_gu,
-    uint16_t* __restrict__ h, float alpha, float limit) {
-  __shared__ __align__(16) uint8_t lds[3 * kAStage + 4 * 4 * kWScBytes];
+    uint8_t* __restrict__ hq, float alpha, float limit) {
+  __shared__ __align__(16) uint8_t lds[3 * kQStage + 4 * 4 * kWScBytes];
   int ti, y;
   xcd_tile<kGuSlots>(blockIdx.x, ti, y);
   const int nt_all = *ntiles;
@@ -412,19 +537,22 @@ __global__ __launch_bounds__(256, 2) void k_prefill_gate_up(
   const long long slot = slot_tab ? slot_tab[gid] : gid;
   const uint8_t* sb = pool + slot * slot_bytes;
   const WSrc src = W == kWT950 ? WSrc{sb, nullptr} : WSrc{sb, sb + kOffGateScales};
-  BRows st;
+  QRows st;
 #pragma unroll
   for (int i = 0; i < 4; ++i)
-    st.rp[i] = x + (long long)(order[tl.p0 + min((tid >> 4) + 16 * i, tl.cnt - 1)] >> 2) * kH;
+    st.rp[i] = xq + (long long)(order[tl.p0 + min((tid >> 4) + 16 * i, tl.cnt - 1)] >> 2) * kQRow;
+  st.srow = xq + (long long)(order[tl.p0 + min(tid & 63, tl.cnt - 1)] >> 2) * kQRow;
   f32x4_t acc[4][4];
   const int ntt = (tl.cnt + 15) >> 4;
-  ptile<W, 4>(src, blk, live, ntt, st, lds, lds + 3 * kAStage + wave * 4 * kWScBytes, acc);
-  // h = bf16(SwiGLU(bf16(acc) + bias)) (the reference's bf16 rounding points) through LDS: oh[row] = the workgroup's
-  // 128 columns.
+  gemm8_tile<W, 4>(src, blk, live, ntt, st, lds, lds + 3 * kQStage + wave * 4 * kWScBytes, acc);
+  // h = bf16(SwiGLU(bf16(acc) + bias)) (the reference's bf16 rounding points), quantised per (row, 32-column block)
+  // into LDS: oh[row] = hi codes of the workgroup's 128 columns | lo codes, os[row] = 4 hi | 4 lo scale bytes.
   uint8_t* oh = lds;
+  uint8_t* os = lds + kPBM * kOhPitch;
   if (live) {
     const uint16_t* bg = bias_gu ? bias_gu + gid * kGU : nullptr;
     float bgv[2], buv[2];
+    uint32_t sh_own = 0, sl_own = 0;
 #pragma unroll
     for (int hb = 0; hb < 2; ++hb) {
       const int j = 16 * (jl + hb) + n;
@@ -447,35 +575,74 @@ __global__ __launch_bounds__(256, 2) void k_prefill_gate_up(
         rb2(g[0], g[1]);
         rb2(u[0], u[1]);
         swiglu_clamp_bf16_2(g, u, alpha, limit, hv);
-        const uint32_t h2 = pack_bf16x2(hv[0], hv[1]);
-        uint8_t* o = oh + (16 * tt + 4 * q + r) * kOhPitch + 2 * (32 * wave + n);
-        *reinterpret_cast<uint16_t*>(o) = (uint16_t)h2;
-        *reinterpret_cast<uint16_t*>(o + 32) = (uint16_t)(h2 >> 16);
+        const uint32_t mx = max(__float_as_uint(hv[0]) & 0x7fffffffu, __float_as_uint(hv[1]) & 0x7fffffffu);
+        const uint32_t sh = x8_scale_byte(__uint_as_float(row16_umax(mx)));
+        const float s_hi = e8m0_f32(sh);
+        fp8x2_t o2 = {0, 0};
+        o2 = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(o2, hv[0], hv[1], s_hi, false);
+        const uint32_t hc = __builtin_bit_cast(uint32_t, o2);
+        const auto d = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(hc, s_hi, false);
+        const float r0 = hv[0] - d[0], r1 = hv[1] - d[1];
+        const uint32_t mr = row16_umax(__float_as_uint(fmaxf(fabsf(r0), fabsf(r1))));
+        const uint32_t sl = x8_scale_byte(__uint_as_float(mr));
+        fp8x2_t l2 = {0, 0};
+        l2 = __builtin_amdgcn_cvt_scalef32_pk_fp8_f32(l2, r0, r1, e8m0_f32(sl), false);
+        const uint32_t lc = __builtin_bit_cast(uint32_t, l2);
+        const int row = 16 * tt + 4 * q + r, c = 32 * wave + n;
+        oh[row * kOhPitch + c] = (uint8_t)hc;
+        oh[row * kOhPitch + c + 16] = (uint8_t)(hc >> 8);
+        oh[row * kOhPitch + kPKT + c] = (uint8_t)lc;
+        oh[row * kOhPitch + kPKT + c + 16] = (uint8_t)(lc >> 8);
+        if (n == 4 * tt + r) {                         // a select: lane n keeps the scales of its row, written below
+          sh_own = sh;
+          sl_own = sl;
+        }
       }
+    }
+    if ((n >> 2) < ntt) {                              // lane (q, n): row 16 (n / 4) + 4 q + n % 4
+      const int row = 16 * (n >> 2) + 4 * q + (n & 3);
+      os[row * 8 + wave] = (uint8_t)sh_own;
+      os[row * 8 + 4 + wave] = (uint8_t)sl_own;
     }
   }
   __syncthreads();
-  // h rows out: 16-byte pieces of the valid columns (64 in column group 22).
-  const int npc = y == 22 ? 8 : 16;
+  // q rows out: 16-byte pieces of the valid columns (64 in column group 22), scale bytes 4 y .. 4 y + 3 (group 22:
+  // bytes 88, 89 and the zero padding 90..95).
+  const int ncol = y == 22 ? 64 : 128;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int pc = tid + 256 * i, row = pc >> 4, c16 = pc & 15;
-    if (row < tl.cnt && c16 < npc)
-      *reinterpret_cast<uint4*>(h + (long long)(tl.p0 + row) * kI + kPKT * y + 8 * c16) =
-          *reinterpret_cast<const uint4*>(oh + row * kOhPitch + 16 * c16);
+    const int pc = tid + 256 * i, row = pc >> 4, c16 = pc & 15, c8 = c16 & 7;
+    if (row < tl.cnt && 16 * c8 < ncol) {
+      const uint2 a0 = *reinterpret_cast<const uint2*>(oh + row * kOhPitch + 16 * c16);
+      const uint2 a1 = *reinterpret_cast<const uint2*>(oh + row * kOhPitch + 16 * c16 + 8);
+      *reinterpret_cast<uint4*>(hq + (long long)(tl.p0 + row) * kQRow + (c16 >> 3) * kQLo + kPKT * y + 16 * c8) =
+          make_uint4(a0.x, a0.y, a1.x, a1.y);
+    }
+  }
+  if (tid < tl.cnt && tid < kPBM) {
+    uint8_t* dst = hq + (long long)(tl.p0 + tid) * kQRow;
+    const uint32_t sh4 = *reinterpret_cast<const uint32_t*>(os + tid * 8);
+    const uint32_t sl4 = *reinterpret_cast<const uint32_t*>(os + tid * 8 + 4);
+    if (y < 22) {
+      *reinterpret_cast<uint32_t*>(dst + kQSh + 4 * y) = sh4;
+      *reinterpret_cast<uint32_t*>(dst + kQSl + 4 * y) = sl4;
+    } else {
+      *reinterpret_cast<uint2*>(dst + kQSh + 88) = make_uint2(sh4 & 0xffff, 0);
+      *reinterpret_cast<uint2*>(dst + kQSl + 88) = make_uint2(sl4 & 0xffff, 0);
+    }
   }
 }
 
 // down + bias, x routing weight, scattered back to pair order: ys[p][n] = bf16(bf16(bf16(y) + b) * w[p]) with p the
-// pair of sorted position p0 + m.  A = the h rows of the tile (consecutive sorted positions).  Grid: max tiles x 16
+// pair of sorted position p0 + m.  A = the h q rows of the tile (consecutive sorted positions).  Grid: max tiles x 16
 // (xcd_tile<2>); wave w: row blocks 12 y + 3 w + i.
 template <int W>
 __global__ __launch_bounds__(256, 2) void k_prefill_down(
-    const uint16_t* __restrict__ h, const int* __restrict__ order, const PTile* __restrict__ tiles,
+    const uint8_t* __restrict__ hq, const int* __restrict__ order, const PTile* __restrict__ tiles,
     const int* __restrict__ ntiles, const uint16_t* __restrict__ wts, const uint8_t* __restrict__ pool,
     long long slot_bytes, const int64_t* __restrict__ slot_tab, long long expert_base,
     const uint16_t* __restrict__ bias_dn, uint16_t* __restrict__ ys) {
-  __shared__ __align__(16) uint8_t lds[3 * kAStage + 4 * kPNB * kWScBytes];
+  __shared__ __align__(16) uint8_t lds[3 * kQStage + 4 * kPNB * kWScBytes];
   int ti, y;
   xcd_tile<kDnSlots>(blockIdx.x, ti, y);
   const int nt_all = *ntiles;
@@ -491,12 +658,13 @@ __global__ __launch_bounds__(256, 2) void k_prefill_down(
   const uint8_t* sb = pool + slot * slot_bytes;
   const WSrc src = W == kWT950 ? WSrc{sb + kTDownOff, nullptr}
                                : WSrc{sb + kOffDownCodes, sb + kOffGateScales + (long long)kGU * (W == kWRaw ? kGK : kPs4Row)};
-  BRows st;
+  QRows st;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) st.rp[i] = h + (long long)(tl.p0 + min((tid >> 4) + 16 * i, tl.cnt - 1)) * kI;
+  for (int i = 0; i < 4; ++i) st.rp[i] = hq + (long long)(tl.p0 + min((tid >> 4) + 16 * i, tl.cnt - 1)) * kQRow;
+  st.srow = hq + (long long)(tl.p0 + min(tid & 63, tl.cnt - 1)) * kQRow;
   f32x4_t acc[4][kPNB];
   const int ntt = (tl.cnt + 15) >> 4;
-  ptile<W, kPNB>(src, blk, true, ntt, st, lds, lds + 3 * kAStage + wave * kPNB * kWScBytes, acc);
+  gemm8_tile<W, kPNB>(src, blk, true, ntt, st, lds, lds + 3 * kQStage + wave * kPNB * kWScBytes, acc);
   // y = bf16(bf16(bf16(acc) + b) * w[p]) per element, staged as the tile's 64 rows x 192 columns in LDS (the A stages
   // are free after the last k-tile's barrier), then written back with 16-byte stores: one 384-byte piece per pair.
   uint8_t* yt = lds;
@@ -537,7 +705,7 @@ __global__ __launch_bounds__(256, 2) void k_prefill_down(
 // ------------------------------------------------------------------------------- plain GEMM (mxfp4_gemm)
 // out[e][m][n] = bf16(sum_k x[m][k] w_e[n][k]); tiles = E * ceil(M / 64) of 64 rows; column group y, wave w: row
 // blocks 12 y + 3 w + i.
-// The fused layer's tiles on bf16 rows (ptile_mfma).
+// The fused layer's tiles on bf16 rows (ktile_bf16).
 NA_DEVICE void store_tile(uint16_t* out_row0, long long pitch, const f32x4_t (&acc)[4][kPNB], const int (&blk)[kPNB],
                           int m_limit) {
   const int lane = threadIdx.x & 63, q = lane >> 4, n = lane & 15;
@@ -575,7 +743,7 @@ __global__ __launch_bounds__(256, 2) void k_mxfp4_gemm(const uint16_t* __restric
                                                        const uint8_t* __restrict__ scales, long long ss_slot,
                                                        const int64_t* __restrict__ slots, uint16_t* __restrict__ out,
                                                        int N, int xcd_slots) {
-  __shared__ __align__(16) uint8_t lds[3 * kAStage + 4 * kPNB * kWScBytes];
+  __shared__ __align__(16) uint8_t lds[3 * kQStage + 4 * kPNB * kWScBytes];
   const int mt = (M + kPBM - 1) / kPBM;
   int i, y;
   gemm_tile_col(blockIdx.x, xcd_slots, N / kPRows, i, y);
@@ -591,7 +759,7 @@ __global__ __launch_bounds__(256, 2) void k_mxfp4_gemm(const uint16_t* __restric
   for (int i = 0; i < 4; ++i) st.rp[i] = x + (long long)min(m0 + (tid >> 4) + 16 * i, M - 1) * kH;
   f32x4_t acc[4][kPNB];
   const int ntt = (min(M - m0, kPBM) + 15) >> 4;
-  ptile<W, kPNB>(src, blk, true, ntt, st, lds, lds + 3 * kAStage + wave * kPNB * kWScBytes, acc);
+  gemm8_tile<W, kPNB>(src, blk, true, ntt, st, lds, lds + 3 * kQStage + wave * kPNB * kWScBytes, acc);
   store_tile(out + ((long long)e * M + m0) * N, N, acc, blk, M - m0);
 }
 
@@ -603,7 +771,7 @@ __global__ __launch_bounds__(256, 2) void k_mxfp4_gemm_grouped(const uint8_t* __
                                                                const uint8_t* __restrict__ scales, long long ss_slot,
                                                                const int64_t* __restrict__ tiles, int block_m, int N,
                                                                int xcd_slots) {
-  __shared__ __align__(16) uint8_t lds[3 * kAStage + 4 * kPNB * kWScBytes];
+  __shared__ __align__(16) uint8_t lds[3 * kQStage + 4 * kPNB * kWScBytes];
   const int sub = max(block_m / kPBM, 1);              // 64-row sub-tiles per tile, one workgroup each
   int i, y;
   gemm_tile_col(blockIdx.x, xcd_slots, N / kPRows, i, y);
@@ -627,7 +795,7 @@ __global__ __launch_bounds__(256, 2) void k_mxfp4_gemm_grouped(const uint8_t* __
   for (int i = 0; i < 4; ++i) st.rp[i] = x + (long long)min(m0 + (tid >> 4) + 16 * i, r1 - 1) * kH;
   f32x4_t acc[4][kPNB];
   const int ntt = (min(r1 - m0, kPBM) + 15) >> 4;
-  ptile<W, kPNB>(src, blk, true, ntt, st, lds, lds + 3 * kAStage + wave * kPNB * kWScBytes, acc);
+  gemm8_tile<W, kPNB>(src, blk, true, ntt, st, lds, lds + 3 * kQStage + wave * kPNB * kWScBytes, acc);
   store_tile(out + (long long)m0 * N, N, acc, blk, r1 - m0);
 }
 
@@ -682,8 +850,8 @@ static PrefillWs prefill_ws(int T) {
   w.order = 1024;
   w.tiles = align256(w.order + P * 4);
   w.xq = align256(w.tiles + (long long)w.max_tiles * sizeof(PTile));
-  w.h = w.xq;                                          // x is read where it is: no rows of its own here
-  w.ys = align256(w.h + P * kI * 2);
+  w.h = align256(w.xq + (long long)T * kQRow);
+  w.ys = align256(w.h + P * kQRow);
   w.total = align256(w.ys + P * kH * 2);
   return w;
 }
@@ -741,21 +909,24 @@ int na_moe_prefill(const void* x, const int64_t* topk_ids, const void* topk_w, i
   int* ntiles = (int*)(ws + w.ntiles);
   int* order = (int*)(ws + w.order);
   PTile* tiles = (PTile*)(ws + w.tiles);
-  uint16_t* h = (uint16_t*)(ws + w.h);
+  uint8_t* xq = ws + w.xq;
+  uint8_t* hq = ws + w.h;
   uint16_t* ys = (uint16_t*)(ws + w.ys);
   hipEvent_t ev[10] = {};
   if (events)
     for (int i = 0; i < 10; ++i) ev[i] = (hipEvent_t)events[i];
   const int P = 4 * T;
-  launch_p(k_prefill_count, dim3(128), dim3(256), stream, ev[0], ev[1], topk_ids, P, counts);
+  const long long qblocks = ((long long)T * kChunks + 255) / 256;
+  launch_p(k_prefill_count, dim3((unsigned)(128 + qblocks)), dim3(256), stream, ev[0], ev[1], topk_ids, P, counts,
+           (const uint16_t*)x, T, xq);
   launch_p(k_prefill_order, dim3(128), dim3(256), stream, ev[2], ev[3], topk_ids, P, (const int*)counts, order, tiles,
            ntiles);
   const dim3 gg(w.max_tiles * 8 * kGuSlots), gd(w.max_tiles * 8 * kDnSlots), blk(256);
 #define NA_PREFILL_GEMMS(W)                                                                                          \
-  launch_p(k_prefill_gate_up<W>, gg, blk, stream, ev[4], ev[5], (const uint16_t*)x, (const int*)order,               \
+  launch_p(k_prefill_gate_up<W>, gg, blk, stream, ev[4], ev[5], (const uint8_t*)xq, (const int*)order,                \
            (const PTile*)tiles, (const int*)ntiles, (const uint8_t*)pool, slot_bytes, slot_tab, expert_base,          \
-           (const uint16_t*)bias_gu, h, alpha, limit);                                                                \
-  launch_p(k_prefill_down<W>, gd, blk, stream, ev[6], ev[7], (const uint16_t*)h, (const int*)order,                    \
+           (const uint16_t*)bias_gu, hq, alpha, limit);                                                                \
+  launch_p(k_prefill_down<W>, gd, blk, stream, ev[6], ev[7], (const uint8_t*)hq, (const int*)order,                    \
            (const PTile*)tiles, (const int*)ntiles, (const uint16_t*)topk_w, (const uint8_t*)pool, slot_bytes,        \
            slot_tab, expert_base, (const uint16_t*)bias_dn, ys);
   if (layout == kWT950) {
