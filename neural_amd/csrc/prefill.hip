@@ -742,11 +742,12 @@ __global__ __launch_bounds__(256, 2) void k_mxfp4_gemm(const uint16_t* __restric
                                                        const uint8_t* __restrict__ blocks, long long sb_slot,
                                                        const uint8_t* __restrict__ scales, long long ss_slot,
                                                        const int64_t* __restrict__ slots, uint16_t* __restrict__ out,
-                                                       int N, int xcd_slots) {
+                                                       int N, int xcd_slots, int tile0) {
   __shared__ __align__(16) uint8_t lds[3 * kQStage + 4 * kPNB * kWScBytes];
   const int mt = (M + kPBM - 1) / kPBM;
   int i, y;
   gemm_tile_col(blockIdx.x, xcd_slots, N / kPRows, i, y);
+  i += tile0;
   if (y >= N / kPRows) return;
   const int e = i / mt, m0 = (i - e * mt) * kPBM;
   const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -856,13 +857,17 @@ static PrefillWs prefill_ws(int T) {
   return w;
 }
 
-// Grid of the GEMM entry points over `tiles` x N / 192 column groups (gemm_tile_col): the XCD order where its 8 x slots
-// column groups are at least 7/8 in use (N = 5760: 30 of 32, N = 2880: 15 of 16), else the plain order.
-static long long gemm_grid(long long tiles, int N, int& xcd_slots) {
+// Grid of the GEMM entry points (gemm_tile_col): workgroups per tile of N / 192 column groups, in the XCD order where
+// its 8 x slots column groups are at least 7/8 in use (N = 5760: 30 of 32, N = 2880: 15 of 16), else the plain order.
+static int gemm_wgs_per_tile(int N, int& xcd_slots) {
   const int cols = N / kPRows, slots = (cols + 7) / 8;
   xcd_slots = 8 * cols >= 7 * 8 * slots ? slots : 0;
-  return tiles * (xcd_slots ? 8 * slots : cols);
+  return xcd_slots ? 8 * slots : cols;
 }
+
+// Workgroups of 256 threads in one launch: a grid dimension holds fewer than 2^32 threads.  The entry points launch
+// more tiles than that in several grids (1,048,576 one-row tiles of 2,880 columns, say).
+constexpr long long kMaxWgs = 0xffffffffLL / 256;
 
 template <typename... KArgs, typename... Args>
 static void launch_p(void (*kern)(KArgs...), dim3 grid, dim3 block, hipStream_t stream, hipEvent_t e0, hipEvent_t e1,
@@ -951,12 +956,14 @@ int na_mxfp4_gemm(const void* x, int M, int K, const void* blocks, long long sb_
   const long long mt = (M + kPBM - 1) / kPBM;
   if (mt * E > 0x7fffffff) return kErrTooLarge;
   int xcd_slots;
-  const long long wgs = gemm_grid(mt * E, N, xcd_slots);
-  if (wgs > 0x7fffffff) return kErrTooLarge;
-  const dim3 grid((unsigned)wgs), blk(256);
+  const int per = gemm_wgs_per_tile(N, xcd_slots);
+  const long long all = mt * E, step = kMaxWgs / per;
+  if (step == 0) return kErrTooLarge;
   auto kern = layout == kWT950 ? k_mxfp4_gemm<kWT950> : layout == kWPs4 ? k_mxfp4_gemm<kWPs4> : k_mxfp4_gemm<kWRaw>;
-  hipLaunchKernelGGL(kern, grid, blk, 0, stream, (const uint16_t*)x, M, (const uint8_t*)blocks, sb_slot,
-                     (const uint8_t*)scales, ss_slot, slots, (uint16_t*)out, N, xcd_slots);
+  for (long long t0 = 0; t0 < all; t0 += step)
+    hipLaunchKernelGGL(kern, dim3((unsigned)(min(step, all - t0) * per)), dim3(256), 0, stream, (const uint16_t*)x, M,
+                       (const uint8_t*)blocks, sb_slot, (const uint8_t*)scales, ss_slot, slots, (uint16_t*)out, N,
+                       xcd_slots, (int)t0);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 
@@ -967,13 +974,14 @@ int na_mxfp4_gemm_grouped(const void* blocks, long long sb_slot, const void* sca
   if (block_m < 16 || (block_m & (block_m - 1)) || block_m > 4096) return kErrArgs;
   if (ntiles == 0) return kOk;
   int xcd_slots;
-  const long long wgs = gemm_grid((long long)ntiles * max(block_m / kPBM, 1), N, xcd_slots);
-  if (wgs > 0x7fffffff) return kErrTooLarge;
-  const dim3 grid((unsigned)wgs), blk(256);
+  const long long per = (long long)gemm_wgs_per_tile(N, xcd_slots) * max(block_m / kPBM, 1), step = kMaxWgs / per;
+  if (step == 0) return kErrTooLarge;
   auto kern = layout == kWT950 ? k_mxfp4_gemm_grouped<kWT950>
             : layout == kWPs4 ? k_mxfp4_gemm_grouped<kWPs4> : k_mxfp4_gemm_grouped<kWRaw>;
-  hipLaunchKernelGGL(kern, grid, blk, 0, stream, (const uint8_t*)blocks, sb_slot, (const uint8_t*)scales, ss_slot,
-                     tiles, block_m, N, xcd_slots);
+  for (long long t0 = 0; t0 < ntiles; t0 += step)
+    hipLaunchKernelGGL(kern, dim3((unsigned)(min(step, ntiles - t0) * per)), dim3(256), 0, stream,
+                       (const uint8_t*)blocks, sb_slot, (const uint8_t*)scales, ss_slot, tiles + 5 * t0, block_m, N,
+                       xcd_slots);
   return hipGetLastError() == hipSuccess ? kOk : kErrLaunch;
 }
 

@@ -76,3 +76,24 @@ def test_grouped_sub_tiles(slots, block_m):
     for i, (x, o) in enumerate(zip(xs, outs)):
         _check(o.float().cpu().numpy().astype(np.float64), x.float().numpy().astype(np.float64),
                slots[1][i % 2][:n], (block_m, i))
+
+
+def test_more_tiles_than_one_grid_holds(slots):
+    """Tiles past 2^32 threads of one grid: 1,048,584 one-row tiles of 16 column groups, and 16,400 grouped tiles of
+    4,096 rows (64 x 16 workgroups each); every row equals the same row of a small call, bit for bit."""
+    import torch
+    from neural_amd.q80 import mxfp4_kernels as mk
+    n = 2880
+    gb, gs = _views(slots, False, n, False)
+    x = synth.bf16_normal(np.random.default_rng(5), (1, n)).cuda()
+    two = mk.mxfp4_gemm(x, gb, gs, torch.tensor([0, 1], device="cuda"))[:, 0]
+    E = 1_048_576 + 8
+    print(f"case gemm E={E} M=1", flush=True)
+    got = mk.mxfp4_gemm(x, gb, gs, torch.arange(E, device="cuda") % 2).view(E // 2, 2, n)
+    assert all(torch.equal(c, two.expand_as(c)) for c in got.split(1 << 16))
+    del got
+    P = 16_400
+    out = torch.full((P, 1, n), 7.0, dtype=torch.bfloat16, device="cuda")
+    print(f"case grouped pairs={P} block_m=4096", flush=True)
+    mk.mxfp4_gemm_grouped_into([(x, i % 2, out[i]) for i in range(P)], gb, gs, block_m=4096)
+    assert torch.equal(out.view(P // 2, 2, n), two.expand(P // 2, 2, n))
