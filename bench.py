@@ -325,7 +325,7 @@ def cpu_prefill_baseline(pool_dev, ids, w, x, threads, seconds):
 def bench_prefill(A):
     """Configuration 2: one MoE layer over T = 2048 prompt tokens (hidden 2880, 128 experts, top-4, Zipf(1.1) expert
     popularity), weights MXFP4 as configuration 0 in the t950 pool, x bf16 N(0,1), zero biases.  One step = the fused
-    prefill layer (five launches), captured in a hipGraph.  Reported: tokens/s, the layer's TFLOP/s on the bf16
+    prefill layer (four launches), captured in a hipGraph.  Reported: tokens/s, the layer's TFLOP/s on the bf16
     MFMA path, and the roofline fraction max(flop / 2.5 PF bf16, bytes / 8 TB/s) / measured time."""
     import torch
 
@@ -378,14 +378,14 @@ def bench_prefill(A):
     for e in ev:
         e.record()
     torch.cuda.synchronize()
-    names = ("count", "order", "gate_up", "down", "combine")
+    names = {"route": 0, "gate_up": 2, "down": 3, "combine": 4}     # launch -> its pair of events
     per = {nm: 0.0 for nm in names}
     R = 5
     for _ in range(R):
         queue_behind_spin(torch)
         rx.forward_prefill(0, x, ids, wts, out=out, events=ev)
         torch.cuda.synchronize()
-        for i, nm in enumerate(names):
+        for nm, i in names.items():
             per[nm] += ev[2 * i].elapsed_time(ev[2 * i + 1]) * 1e3 / R
     P = int(counts.sum())
     flop = 2.0 * P * (5760 * 2880 + 2880 * 2880)

@@ -251,14 +251,15 @@ long long na_moe_prefill_workspace_bytes(int T);
 int na_moe_prefill_workspace_layout(int T, long long* offsets);
 
 /* One MoE layer over T prompt tokens, all experts resident.  Replaces server.py:1837-1936 (moe_prefill) with the
- * expert products of _expert_gemms :1977-2040 for resident experts; five launches: pair counts (with x quantised
- * into exact E4M3 hi + lo rows), stable expert order + 64-token tiles, gate_up + bias + clamped SwiGLU on the
+ * expert products of _expert_gemms :1977-2040 for resident experts; four launches: pair counts, stable expert order and
+ * 64-token tiles (beside x quantised into exact E4M3 hi + lo rows), gate_up + bias + clamped SwiGLU on the
  * block-scaled FP8 x FP4 MFMA (h out as E4M3 hi + lo rows), down + bias + routing weight, top-k sum.
  *   x [T, 2880] bf16; topk_ids int64 [T, 4] (ids outside [0, 128) contribute +0); topk_w bf16 [T, 4]
  *   pool / slot_bytes / slot_tab / expert_base / biases as na_moe_decode; layout 0 raw, 1 PS4, 2 t950
  *   workspace: na_moe_prefill_workspace_bytes(T) bytes, 16-byte aligned
  *   out [T, 2880] bf16 = bf16(sum_k fp32(yw[t, k])) in top-k order
- *   events  NULL or 10 hipEvent_t (start/stop of the five launches) */
+ *   events  NULL or 10 hipEvent_t (start/stop of each launch: routing, -, gate_up, down, top-k sum; events 2
+ *           and 3 are recorded behind the routing launch) */
 int na_moe_prefill(const void* x, const int64_t* topk_ids, const void* topk_w, int T, const void* pool,
                    long long slot_bytes, int layout, const int64_t* slot_tab, long long expert_base,
                    const void* bias_gu, const void* bias_dn, void* workspace, long long ws_bytes, void* out,

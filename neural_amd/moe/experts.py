@@ -173,11 +173,12 @@ class ResidentExperts:
         """Prompt tokens of one layer (the reference's moe_prefill, server.py:1837-1936, for an all-resident pool):
         hidden [T, 2880] bf16, router_indices [T, 4] int64, routing_weights [T, 4] bf16 -> [T, 2880] bf16 =
         per token bf16(sum_k bf16(bf16(expert_k(h) + b_dn) * w_k)) in top-k order, each expert product the
-        reference's GEMM arithmetic.  Five launches on the current stream, no host synchronisation: pair counts per
-        expert, a stable expert-major order of the pairs with its 64-token tiles, gate_up + bias + clamped SwiGLU
+        reference's GEMM arithmetic.  Four launches on the current stream, no host synchronisation: pair counts per
+        expert and a stable expert-major order of the pairs with its 64-token tiles, gate_up + bias + clamped SwiGLU
         (activation rows gathered through the order), down + bias + routing weight (scattered back to pair order),
         and the top-k sum.  The workspace (~ T x 53 KB) is allocated through torch's caching allocator.
-        events: None or ten recorded timing events (start/stop of each launch; measurement only)."""
+        events: None or ten recorded timing events (start/stop of routing, of nothing, of gate_up, down and
+        the sum; measurement only)."""
         L = self.layout
         T = hidden.shape[0]
         if hidden.dtype is not torch.bfloat16 or hidden.ndim != 2 or hidden.shape[1] != L.hidden \

@@ -163,3 +163,30 @@ def test_prefill_raw_ps4_t950_bitwise_at_2048(pools):
     w_d = torch.from_numpy(w).to(torch.bfloat16).to(dev)
     outs = {nm: _run(pools, nm, x, ids_d, w_d)[0] for nm in ("raw", "ps4", "t950")}
     assert torch.equal(outs["raw"], outs["t950"]) and torch.equal(outs["ps4"], outs["t950"])
+
+
+@pytest.mark.parametrize("T,kind", [(1, "zipf"), (16, "none"), (23, "zipf"), (513, "one"), (2049, "zipf"), (2049, "one")])
+def test_prefill_routing_tables_small_and_uneven(pools, T, kind):
+    """The routing launch at one pair step, a few, and one pair past a round of 8,192; every pair in one expert's list
+    ("one": the four ranks alike, which the layer accepts) and no valid pair at all ("none")."""
+    import torch
+    from neural_amd import synth
+    dev = pools["dev"]
+    print(f"case prefill routing tables T={T} {kind}", flush=True)
+    rng = np.random.default_rng(T)
+    ids, w = synth.zipf_routing(rng, T)
+    if kind != "zipf":
+        ids = np.full_like(ids, 127 if kind == "one" else -1)
+    x = synth.bf16_normal(rng, (T, H)).to(dev)
+    out, ws, offs = _run(pools, "t950", x, torch.from_numpy(ids).to(dev), torch.from_numpy(w).to(torch.bfloat16).to(dev))
+    counts, ntiles, order, tiles = _tables(ws, offs, 4 * T)
+    flat = ids.reshape(-1)
+    valid = (flat >= 0) & (flat < NE)
+    want = np.bincount(flat[valid], minlength=NE)
+    assert np.array_equal(counts, want)
+    assert np.array_equal(order[:valid.sum()], np.argsort(np.where(valid, flat, NE), kind="stable")[:valid.sum()])
+    start = np.cumsum(want) - want
+    rows = [(e, start[e] + m0, min(64, want[e] - m0), 0) for e in range(NE) for m0 in range(0, want[e], 64)]
+    assert ntiles == len(rows) and np.array_equal(tiles, np.array(rows, np.int32).reshape(-1, 4))
+    if kind == "none":
+        assert not bool(out.float().abs().sum())
