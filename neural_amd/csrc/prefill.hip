@@ -292,9 +292,11 @@ struct WScales {
 };
 
 // One wave's weight stream over its NB row blocks: the code bytes of a k-tile, one 16-byte load per lane and row block
-// in the MFMA's operand order, at 32-bit offsets from the matrix (lane (q, n): t950 the 16 bytes at 1024 t + 16 lane of
-// the block, raw / PS4 those of group 4t + q of row n; groups 90, 91 re-read group 89 and are zeroed at the use).  The
-// E8M0 rows of the blocks are staged once in the wave's LDS area wsc (load_scales, store_scales) and read per k-tile from there.
+// in the MFMA's operand order (lane (q, n): t950 the 16 bytes at 1024 t + 16 lane of the block, raw / PS4 those of group
+// 4t + q of row n; groups 90, 91 re-read group 89 and are zeroed at the use).  The block's own offset is 64-bit and
+// wave-uniform (the GEMM entry points take any N: 1.49 M rows of codes pass 2^31 bytes), the lane's within it 32-bit.
+// The E8M0 rows of the blocks are staged once in the wave's LDS area wsc (load_scales, store_scales) and read per k-tile
+// from there.
 template <int W, int NB>
 struct WStream {
   WSrc src;
@@ -310,7 +312,8 @@ struct WStream {
       if constexpr (W == kWT950)
         c[nb] = load16(src.codes + (long long)blk[nb] * kTBlock + t * 1024 + 16 * lane);
       else
-        c[nb] = load16(src.codes + (uint32_t)((blk[nb] * 16 + (lane & 15)) * kRowBytes + 16 * g));
+        c[nb] = load16(src.codes + (long long)blk[nb] * (kTRows * kRowBytes) +
+                       (uint32_t)((lane & 15) * kRowBytes + 16 * g));
     }
   }
   // The blocks' scale rows through registers to LDS, by 16-byte pieces: the loads are issued before the first k-tiles'

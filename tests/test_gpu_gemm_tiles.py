@@ -97,3 +97,34 @@ def test_more_tiles_than_one_grid_holds(slots):
     print(f"case grouped pairs={P} block_m=4096", flush=True)
     mk.mxfp4_gemm_grouped_into([(x, i % 2, out[i]) for i in range(P)], gb, gs, block_m=4096)
     assert torch.equal(out.view(P // 2, 2, n), two.expand(P // 2, 2, n))
+
+
+@pytest.mark.parametrize("packed", [False, True])
+def test_codes_past_32_bit_offsets(packed):
+    """Row blocks on both sides of 2^31 and 2^32 code bytes (1,440 a row), and the last one: the same bits, bit for bit,
+    as the product with those 192 rows alone.  The reference product of the rows just past 4 GiB is checked in 64 bits."""
+    import torch
+    from neural_amd.q80 import mxfp4_kernels as mk
+    n = 192 * (2 ** 32 // (192 * 1440) + 2)
+    w = 46 if packed else 90
+    print(f"case gemm N={n} packed={packed}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(17)
+    codes = torch.empty(n * 1440 // 8, dtype=torch.int64, device="cuda").random_(generator=g).view(torch.uint8)
+    codes = codes.view(1, n, 90, 16)
+    scales = torch.randint(0 if packed else 119, 126, (1, n, w), generator=g, dtype=torch.uint8, device="cuda")
+    if packed:
+        scales[:, :, 0] = 119                           # base byte; the others hold two 4-bit deltas each
+        scales[:, :, 1:] &= 0x33
+    x = synth.bf16_normal(np.random.default_rng(6), (5, 2880)).cuda()
+    slot = torch.zeros(1, dtype=torch.int64, device="cuda")
+    full = mk.mxfp4_gemm(x, codes, scales, slot)[0]
+    out = torch.empty_like(full)
+    mk.mxfp4_gemm_grouped_into([(x, 0, out)], codes, scales)
+    assert torch.equal(full, out)
+    for r0 in (0, 2 ** 31 // 1440 // 192 * 192, 2 ** 32 // 1440 // 192 * 192, n - 192):
+        cb, sb = codes[:, r0:r0 + 192].clone(), scales[:, r0:r0 + 192].clone()
+        assert torch.equal(full[:, r0:r0 + 192], mk.mxfp4_gemm(x, cb, sb, slot)[0]), r0
+    sc = sb[0].cpu().numpy()
+    wts = mo.dequant_rows(cb[0].cpu().numpy(), mo.ps4_unpack_rows(sc) if packed else sc).astype(np.float64)
+    _check(full[:, n - 192:].float().cpu().numpy().astype(np.float64), x.float().cpu().numpy().astype(np.float64), wts,
+           (packed, n))
