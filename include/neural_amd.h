@@ -226,7 +226,10 @@ int na_ring_write(void* kc, void* vc, int ring, const void* k_new, const void* v
  *   x        bf16 [M, K], K = 2880 (16-byte aligned rows)
  *   blocks   layout 0 (raw) / 1 (PS4): u8 view [cap, N, 90, 16], slot stride sb_slot; scales [cap, N, 90 | 46] with
  *            slot stride ss_slot.  layout 2: blocks = the matrix's first t950 row block of slot 0, stride sb_slot.
- *   out      bf16 [E, M, N], N a multiple of 192 */
+ *   out      bf16 [E, M, N], N a multiple of 192
+ * Products are exact for every scale byte 0 .. 254 (a weight past bf16's range, at bytes 253 and 254, keeps its finite
+ * product with a small x); byte 255 gives NaN.  An infinite x gives infinities of the products' signs, and NaN where it
+ * meets a weight of zero or products of both signs; a NaN gives NaN. */
 int na_mxfp4_gemm(const void* x, int M, int K, const void* blocks, long long sb_slot, const void* scales,
                   long long ss_slot, int layout, const int64_t* slots, int E, void* out, int N, hipStream_t stream);
 

@@ -12,7 +12,7 @@
 // states the quantiser).
 //
 // The plain and grouped GEMM entry points (bf16 activations, no workspace) run the same tiles on bf16 rows and
-// v_mfma_f32_16x16x32_bf16, the weights converted to bf16 (exact) in registers.  They are HBM-bound where experts have
+// v_mfma_f32_16x16x32_bf16, the weights converted to bf16 (exact; gemm8_wide past bf16's range) in registers.  They are HBM-bound where experts have
 // few rows: 2,000 Zipf-routed rows over a raw store, gate_up and down, 1,390 -> 493 us (1.7 GB) when the scales went
 // through LDS instead of scattered byte loads, tiles stopped staging and multiplying their empty 16-row blocks, column
 // groups got the XCD order, and the kernels, 400 registers before, came to fit two workgroups per CU; 493 -> 462 us,
@@ -42,11 +42,22 @@ struct WSrc {
 };
 
 // Two E2M1 codes of byte SEL of `word`, times 2^e of the float `scale` -> packed bf16 pair (low nibble = element 0 in the
-// low half): exact for every E8M0 scale byte up to 252 (byte 0 is 2^-127).  At 253 (codes of 4 and 6) and 254 (codes of 2
-// and above) a weight is past bf16's range and infinite, as in the reference's dequantisation to bf16.
+// low half): exact for every E8M0 scale byte up to 252 (byte 0, the float 0, is 2^-127), NaN at 255.
 template <int SEL>
 NA_DEVICE uint32_t fp4x2_scaled(uint32_t word, float scale) {
   return __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(word, scale, SEL));
+}
+
+// Scale bytes from which a weight can be past bf16's largest value: codes of 4 and 6 at 253, of 2 and above at 254.
+constexpr uint32_t kE8m0Wide = 253;
+
+// A quarter of the same two weights from the scale byte: exact for every byte up to 254 (2^-130 .. 1.5 x 2^127), NaN at
+// 255.
+template <int SEL>
+NA_DEVICE uint32_t fp4x2_quarter(uint32_t word, uint32_t byte) {
+  const auto v = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(word, 1.0f, SEL);
+  const int e = (int)byte - 129;
+  return byte == 255 ? 0x7fc07fc0u : pack_bf16x2(__builtin_amdgcn_ldexpf(v[0], e), __builtin_amdgcn_ldexpf(v[1], e));
 }
 
 constexpr int kPNB = 3;                  // row blocks per wave in the plain, grouped and down kernels
@@ -256,6 +267,14 @@ struct BRows {
   template <int NT>
   using Stage = BStage<NT>;
   const uint16_t* rp[4];
+  const uint16_t* x0;                                  // staged row r: row min(r, last) of x0
+  int last;
+
+  NA_DEVICE BRows(const uint16_t* x0_, int last_, int tid) : x0(x0_), last(last_) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) rp[i] = row((tid >> 4) + 16 * i);
+  }
+  NA_DEVICE const uint16_t* row(int r) const { return x0 + min(r, last) * kH; }
 
   template <int NT>
   NA_DEVICE void load(int t, int tid, BStage<NT>& a) const {
@@ -304,6 +323,7 @@ struct WStream {
   uint8_t* wsc;
   int lane;
   int base[NB];                                        // PS4: base byte of this lane's row, per row block
+  uint32_t top;                                        // bf16 rows: this lane's largest scale byte (gemm8_wide)
 
   NA_DEVICE void load(int t, uint4 (&c)[NB]) const {
     const int g = min(4 * t + (lane >> 4), kGK - 1);
@@ -400,7 +420,7 @@ NA_DEVICE void ktile_x8(int t, const WStream<W, NB>& ws, const uint8_t* cur, con
 // k-tile of a full tile against the 48 conversions).  MFMA j multiplies elements 8 j .. 8 j + 7 of each of the k-tile's
 // four 32-element groups (lane 16 kb + m: group kb), on both operands.
 template <int W, int NB, int NT>
-NA_DEVICE void ktile_bf16(int t, const WStream<W, NB>& ws, const uint8_t* cur, const uint4 (&c)[NB],
+NA_DEVICE void ktile_bf16(int t, WStream<W, NB>& ws, const uint8_t* cur, const uint4 (&c)[NB],
                           f32x4_t (&acc)[4][NB]) {
   const int lane = threadIdx.x & 63, kb = lane >> 4, m = lane & 15;
   uint4 b[NB][4];
@@ -408,7 +428,9 @@ NA_DEVICE void ktile_bf16(int t, const WStream<W, NB>& ws, const uint8_t* cur, c
   for (int nb = 0; nb < NB; ++nb) {
     const bool in = 4 * t + kb < kGK;
     const uint32_t w[4] = {in ? c[nb].x : 0u, in ? c[nb].y : 0u, in ? c[nb].z : 0u, in ? c[nb].w : 0u};
-    const float s = e8m0_f32((uint32_t)ws.scale(t, nb) & 0xff);
+    const uint32_t sb = (uint32_t)ws.scale(t, nb) & 0xff;
+    ws.top = max(ws.top, sb);
+    const float s = e8m0_f32(sb);
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       b[nb][j] = make_uint4(fp4x2_scaled<0>(w[j], s), fp4x2_scaled<1>(w[j], s), fp4x2_scaled<2>(w[j], s),
@@ -433,7 +455,7 @@ NA_DEVICE void ktile_bf16(int t, const WStream<W, NB>& ws, const uint8_t* cur, c
 // issues the loads of A of k-tile t + 2 (into a_in) and of the weights of k-tile t + 2 (into c2), runs the
 // MFMAs, stores A of k-tile t + 1 (loaded one step earlier, a_out) at nxt and meets the barrier.
 template <int W, int NB, int NT, typename S>
-NA_DEVICE void gemm8_step(int t, const WStream<W, NB>& ws, bool live, const S& st, const uint8_t* cur, uint8_t* nxt,
+NA_DEVICE void gemm8_step(int t, WStream<W, NB>& ws, bool live, const S& st, const uint8_t* cur, uint8_t* nxt,
                           const typename S::template Stage<NT>& a_out, typename S::template Stage<NT>& a_in,
                           const uint4 (&c)[NB], uint4 (&c2)[NB], f32x4_t (&acc)[4][NB]) {
   const int tid = threadIdx.x;
@@ -467,14 +489,13 @@ NA_DEVICE void gemm8_step(int t, const WStream<W, NB>& ws, bool live, const S& s
 // scale rows).  A wave without work (live = false) stages and meets every barrier but runs no MFMA.  All 256 threads must
 // call it.
 template <int W, int NB, int NT, typename S>
-NA_DEVICE void gemm8_tile_n(const WSrc& src, const int (&blk)[NB], bool live, const S& st, uint8_t* lds, uint8_t* wsc,
+NA_DEVICE void gemm8_tile_n(WStream<W, NB>& ws, bool live, const S& st, uint8_t* lds,
                             f32x4_t (&acc)[4][NB]) {
   const int tid = threadIdx.x, lane = tid & 63;
 #pragma unroll
   for (int tt = 0; tt < 4; ++tt)
 #pragma unroll
     for (int nb = 0; nb < NB; ++nb) acc[tt][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  WStream<W, NB> ws{src, blk, wsc, lane, {}};
   uint4 wsv[NB][WStream<W, NB>::kScRounds];
   ws.load_scales(wsv);
   uint8_t* const b0 = lds;
@@ -501,19 +522,65 @@ NA_DEVICE void gemm8_tile_n(const WSrc& src, const int (&blk)[NB], bool live, co
   gemm8_step<W, NB, NT, S>(t + 1, ws, live, st, b1, b2, a2, a0, c1, c0, acc);   // 22
 }
 
+// acc of gemm8_tile again where one of the wave's scale bytes is kE8m0Wide or more: there a weight may be past bf16's
+// range though its product with a small x is finite, as the scaled instruction and the GEMV have it.  A quarter of every
+// weight is inside the range, and four equal products are added in the place of one.  One wave by itself, without
+// barriers: fragments straight from the rows and codes, scales from the wave's LDS area.  Such bytes (weights of 2^126
+// and more) occur in no trained model, so this is kept small, not fast; the test for them is one maximum per conversion
+// and one branch per tile (a branch per k-tile cost 40 to 90 spilled registers).
+template <int W, int NB>
+NA_DEVICE void gemm8_wide(const WStream<W, NB>& ws, const BRows& st, int ntt, f32x4_t (&acc)[4][NB]) {
+  const int kb = ws.lane >> 4, m = ws.lane & 15;
+#pragma unroll
+  for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) acc[tt][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+  for (int t = 0; t < kPTiles; ++t) {
+    const bool in = 4 * t + kb < kGK;
+    uint4 c[NB];
+    ws.load(t, c);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      bf16x8_t a[4];
+#pragma unroll
+      for (int tt = 0; tt < 4; ++tt) {
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (in && tt < ntt) v = *reinterpret_cast<const uint4*>(st.row(16 * tt + m) + t * kPKT + 32 * kb + 8 * j);
+        a[tt] = __builtin_bit_cast(bf16x8_t, v);
+      }
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        const uint32_t cw[4] = {c[nb].x, c[nb].y, c[nb].z, c[nb].w};
+        const uint32_t w = in ? cw[j] : 0u, sb = (uint32_t)ws.scale(t, nb) & 0xff;
+        const bf16x8_t b = __builtin_bit_cast(bf16x8_t, make_uint4(fp4x2_quarter<0>(w, sb), fp4x2_quarter<1>(w, sb),
+                                                                   fp4x2_quarter<2>(w, sb), fp4x2_quarter<3>(w, sb)));
+#pragma unroll 1
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int tt = 0; tt < 4; ++tt)
+            acc[tt][nb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[tt], b, acc[tt][nb], 0, 0, 0);
+      }
+    }
+  }
+}
+
 // gemm8_tile_n for a tile whose rows fill ntt (1..4) 16-token blocks: empty blocks are neither staged nor multiplied.
 // ntt is workgroup-uniform.
 template <int W, int NB, typename S>
 NA_DEVICE void gemm8_tile(const WSrc& src, const int (&blk)[NB], bool live, int ntt, const S& st, uint8_t* lds,
                           uint8_t* wsc, f32x4_t (&acc)[4][NB]) {
+  WStream<W, NB> ws{src, blk, wsc, (int)(threadIdx.x & 63), {}, 0};
   if (ntt > 3)
-    gemm8_tile_n<W, NB, 4, S>(src, blk, live, st, lds, wsc, acc);
+    gemm8_tile_n<W, NB, 4, S>(ws, live, st, lds, acc);
   else if (ntt == 3)
-    gemm8_tile_n<W, NB, 3, S>(src, blk, live, st, lds, wsc, acc);
+    gemm8_tile_n<W, NB, 3, S>(ws, live, st, lds, acc);
   else if (ntt == 2)
-    gemm8_tile_n<W, NB, 2, S>(src, blk, live, st, lds, wsc, acc);
+    gemm8_tile_n<W, NB, 2, S>(ws, live, st, lds, acc);
   else
-    gemm8_tile_n<W, NB, 1, S>(src, blk, live, st, lds, wsc, acc);
+    gemm8_tile_n<W, NB, 1, S>(ws, live, st, lds, acc);
+  if constexpr (S::kBf16)
+    if (__any(ws.top >= kE8m0Wide)) gemm8_wide<W, NB>(ws, st, ntt, acc);
 }
 
 // Workgroup b -> (tile, column group): the dispatcher deals workgroups to the 8 XCDs in turn (XCD b % 8), so XCD x
@@ -778,9 +845,7 @@ __global__ __launch_bounds__(256, 2) void k_mxfp4_gemm(const uint16_t* __restric
 #pragma unroll
   for (int i = 0; i < kPNB; ++i) blk[i] = y * (4 * kPNB) + kPNB * wave + i;
   const WSrc src = w_src<W>(blocks, sb_slot, scales, ss_slot, slots[e]);
-  BRows st;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) st.rp[i] = x + (long long)min(m0 + (tid >> 4) + 16 * i, M - 1) * kH;
+  const BRows st(x + (long long)m0 * kH, M - 1 - m0, tid);
   f32x4_t acc[4][kPNB];
   const int ntt = (min(M - m0, kPBM) + 15) >> 4;
   gemm8_tile<W, kPNB>(src, blk, true, ntt, st, lds, lds + 3 * kQStage + wave * kPNB * kWScBytes, acc);
@@ -814,9 +879,7 @@ __global__ __launch_bounds__(256, 2) void k_mxfp4_gemm_grouped(const uint8_t* __
 #pragma unroll
   for (int i = 0; i < kPNB; ++i) blk[i] = y * (4 * kPNB) + kPNB * wave + i;
   const WSrc src = w_src<W>(blocks, sb_slot, scales, ss_slot, slot);
-  BRows st;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) st.rp[i] = x + (long long)min(m0 + (tid >> 4) + 16 * i, r1 - 1) * kH;
+  const BRows st(x + (long long)m0 * kH, r1 - 1 - m0, tid);
   f32x4_t acc[4][kPNB];
   const int ntt = (min(r1 - m0, kPBM) + 15) >> 4;
   gemm8_tile<W, kPNB>(src, blk, true, ntt, st, lds, lds + 3 * kQStage + wave * kPNB * kWScBytes, acc);
