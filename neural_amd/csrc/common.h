@@ -212,12 +212,14 @@ NA_DEVICE float wave_total(float v) {
   return (r0 + r1) + (r2 + r3);
 }
 
-// bf16(1 / (1 + exp(-t))) of a bf16 value t, on the hardware's base-2 exponential and reciprocal (both within 1 fp32
-// ulp): the bits of the correctly rounded fp32 expression at every bf16 t except the three (-87.5, -88, -88.5) whose
-// sigmoid is below 2^-126 and becomes +0 (na_selftest_swiglu, all 65,536 arguments).  expf and the IEEE division took
-// about 25 instructions more per value; the epilogue of a full prompt tile (32 values per lane) was 18 % of it.
-NA_DEVICE float sigmoid_bf16(float t) {
-  return rb(__builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t * -1.44269504f)));
+// fp32 1 / (1 + exp(-t)) of a bf16 value t on the hardware's base-2 exponential and reciprocal, as the quarter of the
+// reciprocal of (1 + e) / 4: v_rcp_f32 gives 0 for a result below 2^-126, which the reciprocal of 1 + e reaches (t = -87.5
+// .. -88.5) and that of its quarter does not.  Each instruction is within 1 fp32 ulp, the value is not: the rounding of
+// t log2(e) grows with |t|, to 54 ulp near -88 (expf and an IEEE division: 2 ulp).  Rounded to bf16, which is all that
+// the callers use, it has the bits of the latter at every one of the 65,536 t (test_gpu_swiglu.py).  expf and the
+// division took about 25 instructions more per value.
+NA_DEVICE float sigmoid_f32(float t) {
+  return 0.25f * __builtin_amdgcn_rcpf(fmaf(__builtin_amdgcn_exp2f(t * -1.44269504f), 0.25f, 0.25f));
 }
 
 // Clamped SwiGLU of one (gate, up) element pair with torch's bf16 op-by-op rounding
@@ -226,7 +228,7 @@ NA_DEVICE float sigmoid_bf16(float t) {
 NA_DEVICE float swiglu_clamp_bf16(float g, float u, float alpha, float limit) {
   const float gate = fminf(g, limit);
   const float up = __builtin_amdgcn_fmed3f(u, -limit, limit);
-  const float s = sigmoid_bf16(rb(gate * alpha));
+  const float s = rb(sigmoid_f32(rb(gate * alpha)));
   const float glu = rb(gate * s);
   return rb(rb(up + 1.0f) * glu);
 }
@@ -243,7 +245,7 @@ NA_DEVICE void swiglu_clamp_bf16_2(const float (&g)[2], const float (&u)[2], flo
   rb2(t[0], t[1]);
   rb2(up[0], up[1]);
 #pragma unroll
-  for (int i = 0; i < 2; ++i) s[i] = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t[i] * -1.44269504f));
+  for (int i = 0; i < 2; ++i) s[i] = sigmoid_f32(t[i]);
   rb2(s[0], s[1]);
 #pragma unroll
   for (int i = 0; i < 2; ++i) s[i] *= gate[i];
