@@ -222,12 +222,15 @@ NA_DEVICE float sigmoid_f32(float t) {
   return 0.25f * __builtin_amdgcn_rcpf(fmaf(__builtin_amdgcn_exp2f(t * -1.44269504f), 0.25f, 0.25f));
 }
 
+// min(max(u, -limit), limit) in one instruction, NaN included: with the lower bound at most the upper one, so
+// that a negative limit (the store-layout and prompt entry points take any) gives the limit as the two steps do.
+NA_DEVICE float clamp_up(float u, float limit) { return __builtin_amdgcn_fmed3f(u, fminf(-limit, limit), limit); }
+
 // Clamped SwiGLU of one (gate, up) element pair with torch's bf16 op-by-op rounding
 // (reference neural/q80/expert_runtime.py:63-72, server.py:2014-2021): inputs are bf16 values, the result is one.
-// med3(u, -limit, limit) is min(max(u, -limit), limit), NaN included.
 NA_DEVICE float swiglu_clamp_bf16(float g, float u, float alpha, float limit) {
   const float gate = fminf(g, limit);
-  const float up = __builtin_amdgcn_fmed3f(u, -limit, limit);
+  const float up = clamp_up(u, limit);
   const float s = rb(sigmoid_f32(rb(gate * alpha)));
   const float glu = rb(gate * s);
   return rb(rb(up + 1.0f) * glu);
@@ -239,7 +242,7 @@ NA_DEVICE void swiglu_clamp_bf16_2(const float (&g)[2], const float (&u)[2], flo
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     gate[i] = fminf(g[i], limit);
-    up[i] = __builtin_amdgcn_fmed3f(u[i], -limit, limit) + 1.0f;
+    up[i] = clamp_up(u[i], limit) + 1.0f;
     t[i] = gate[i] * alpha;
   }
   rb2(t[0], t[1]);

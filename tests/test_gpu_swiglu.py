@@ -2,7 +2,8 @@
 the oracle.  At the model's alpha and limit: every finite bf16 gate value, with the up values +-0, +-1, the limit and
 beyond it.  With alpha = +-1 and no limit the sigmoid's argument is +-gate: every bf16 argument, the same bits as the fp32
 expression 1 / (1 + exp(-t)) with correctly rounded steps, infinite and NaN gates and ups included (the clamps return the
-other operand for a NaN).  The paired form gives the single form's bits."""
+other operand for a NaN).  A limit below zero is the clamp's result for every up value, as min(max(u, -limit), limit) has
+it.  The paired form gives the single form's bits."""
 import numpy as np
 import pytest
 
@@ -38,7 +39,8 @@ def test_swiglu_every_gate_value():
     assert np.abs(bf16_bits_to_f32(got)[tiny].astype(np.float64) - want[tiny]).max() < 2.0 ** -120 * 8
 
 
-@pytest.mark.parametrize("alpha,limit", [(1.0, np.inf), (-1.0, np.inf), (1.702, 7.0)])
+# No limit of 0: the minimum of two zeros of opposite sign may be either (numpy's and the hardware's differ).
+@pytest.mark.parametrize("alpha,limit", [(1.0, np.inf), (-1.0, np.inf), (1.702, 7.0), (1.702, -3.0)])
 def test_swiglu_every_sigmoid_argument(alpha, limit):
     import torch
     from neural_amd import _native as N
