@@ -352,19 +352,6 @@ __global__ __launch_bounds__(256) void k_oproj(const uint16_t* __restrict__ att,
   oproj_body<TPR, false>(blockIdx.x, hc, att, Wo, bo, xbuf, nullptr, nullptr, mid, nullptr, nullptr, 0, nullptr);
 }
 
-// post-attention RMSNorm + router + top-4: 256 / TPR experts per workgroup, grid 128 / (256 / TPR).  Workgroup 0 writes hn (the experts' input);
-// every workgroup publishes its 16 logits (device-coherent stores, then a count); the last one selects the top 4,
-// writes ids / weights and resets the count.
-// Router phase: NR = 128 / (256 / TPR) workgroups; workgroup `blk` computes 256 / TPR logits.  FUSED (the last phase
-// of k_attn_block): the weights and the norm weight are loaded first, then thread 0 polls one tagged word of mid
-// (mid_tags; gen: the generation word as loaded at entry) and every thread reads its 8 words.  With ids (select):
-// the logits are also written as tagged words (logit_tags), and the last workgroup (blk = NR - 1) reads all 128 of
-// them, selects the top 4 and stores gen into *gen_word: every workgroup of the launch has read the old number by
-// then (each one's result is an input of the router's logits, and each read the number before it produced
-// anything).  Without ids the logits go to `logits` only, for the next launch (the expert body selects the top 4
-// itself): each workgroup counts itself into *entered once its read of the generation word is complete, and the
-// last workgroup, once its own logits are stored, waits for all NR counts (the other phases' workgroups have read
-// the word, since their results fed its mid), returns the count to zero and advances the word.
 // The serving outputs that na_core_router_pack adds to the router's (k_route_pack states them).
 struct RoutePack {
   const int64_t* slot_tab;
@@ -416,6 +403,19 @@ NA_DEVICE void route_pack_near(const RoutePack& rp, int lane, float v0, float v1
   }
 }
 
+// post-attention RMSNorm + router + top-4: 256 / TPR experts per workgroup, grid 128 / (256 / TPR).  Workgroup 0 writes
+// hn (the experts' input); every workgroup publishes its 256 / TPR logits (device-coherent stores, then a count); the
+// last one selects the top 4, writes ids / weights and resets the count.
+// Router phase: NR = 128 / (256 / TPR) workgroups; workgroup `blk` computes 256 / TPR logits.  FUSED (the last phase
+// of k_attn_block): the weights and the norm weight are loaded first, then thread 0 polls one tagged word of mid
+// (mid_tags; gen: the generation word as loaded at entry) and every thread reads its 8 words.  With ids (select):
+// the logits are also written as tagged words (logit_tags), and the last workgroup (blk = NR - 1) reads all 128 of
+// them, selects the top 4 and stores gen into *gen_word: every workgroup of the launch has read the old number by
+// then (each one's result is an input of the router's logits, and each read the number before it produced
+// anything).  Without ids the logits go to `logits` only, for the next launch (the expert body selects the top 4
+// itself): each workgroup counts itself into *entered once its read of the generation word is complete, and the
+// last workgroup, once its own logits are stored, waits for all NR counts (the other phases' workgroups have read
+// the word, since their results fed its mid), returns the count to zero and advances the word.
 // rp (not FUSED): the serving outputs, written where their inputs already are: workgroup 0's normed mid, the last
 // workgroup's top 4.
 template <int TPR, bool FUSED>

@@ -13,11 +13,11 @@
 //
 // The plain and grouped GEMM entry points (bf16 activations, no workspace) run the same tiles on bf16 rows and
 // v_mfma_f32_16x16x32_bf16, the weights converted to bf16 (exact; gemm8_wide past bf16's range) in registers.  They are HBM-bound where experts have
-// few rows: 2,000 Zipf-routed rows over a raw store, gate_up and down, 1,390 -> 493 us (1.7 GB) when the scales went
+// few rows: 2,000 Zipf-routed rows over a raw store, gate_up and down (1.7 GB), 1,390 -> 536 us when the scales went
 // through LDS instead of scattered byte loads, tiles stopped staging and multiplying their empty 16-row blocks, column
-// groups got the XCD order, and the kernels, 400 registers before, came to fit two workgroups per CU; 493 -> 462 us,
-// and one expert's 4,096 rows 320 -> 213 us (957 TFLOP/s), when the rows stopped being quantised into hi + lo E4M3
-// rows by every column group.
+// groups got the XCD order, and the kernels, 400 registers before, came to fit two workgroups per CU; -> 493 us with the
+// activation quantiser's one-instruction block maxima; -> 462 us, and one expert's 4,096 rows 320 -> 213 us
+// (957 TFLOP/s), when the rows stopped being quantised into hi + lo E4M3 rows by every column group.
 //
 // Weight layouts (template W): the store's raw and PS4 slots (row r: 1,440 code bytes, then a raw 90-byte or PS4
 // 46-byte scale row; lane (q, n) reads the 16 bytes of group 4t + q of row n, already the MFMA's B order) and the t950
@@ -414,11 +414,11 @@ NA_DEVICE void ktile_x8(int t, const WStream<W, NB>& ws, const uint8_t* cur, con
 }
 
 // The MFMAs of k-tile t on bf16 rows: the E2M1 codes x 2^(s - 127) converted to bf16 (exact), 16 conversions per row
-// block and k-tile shared by the tile's 16-token blocks.  v_mfma_f32_16x16x32_bf16 at half the scaled instruction's
-// rate and one row instead of hi and lo: the same matrix-core time, the reference's exact products, and no
-// quantisation of the rows (which each of the 15 to 30 column groups repeated: about 220 vector instructions per
-// k-tile of a full tile against the 48 conversions).  MFMA j multiplies elements 8 j .. 8 j + 7 of each of the k-tile's
-// four 32-element groups (lane 16 kb + m: group kb), on both operands.
+// block and k-tile shared by the tile's 16-token blocks.  By itself v_mfma_f32_16x16x32_bf16 is the slower exact route
+// (1,546 TFLOP/s when nothing else runs, against 2,391 of the scaled instruction on hi and lo rows); these kernels stay
+// below either, and gain from not quantising their rows, which each of the 15 to 30 column groups repeated: about 220
+// vector instructions per k-tile of a full tile against the 48 conversions.  MFMA j multiplies elements 8 j .. 8 j + 7
+// of each of the k-tile's four 32-element groups (lane 16 kb + m: group kb), on both operands.
 template <int W, int NB, int NT>
 NA_DEVICE void ktile_bf16(int t, WStream<W, NB>& ws, const uint8_t* cur, const uint4 (&c)[NB],
                           f32x4_t (&acc)[4][NB]) {
@@ -594,10 +594,15 @@ NA_DEVICE void xcd_tile(int b, int& tile, int& col) {
   col = SLOTS * (b & 7) + s % SLOTS;
 }
 
-// A full tile's workgroup (stamped, cycles): prologue 8,860 -> 5,900 since the weights, their scales and the row
-// addresses are requested side by side; its 23 k-tiles 2,100 each (1,024 of MFMAs; two workgroups share a SIMD);
-// epilogue 15,700 -> 8,700 (32 activations per lane) by the hardware exponential and reciprocal, block maxima of one
-// instruction per step and shared conversions.  Layer: 2,048 tokens 665 -> 630 us, 23 tokens 191 -> 182, same bits.
+// What bounds it, from stamps of every workgroup (one expert's rows in full tiles, 4 x 1,024 rows, 1,472 workgroups):
+// two workgroups on a CU for 81 % of the launch (1.74 on average: six a CU in three rounds, then a part-empty end), each
+// 77,300 cycles: 5,800 before its first k-tile, 23 k-tiles of 2,616, of which the two waves of a SIMD fill 2,048 with
+// MFMAs, 11,300 of epilogue (32 activations per lane).  The clock is 1.92 GHz under this load (2.2 with one workgroup on
+// a third of the CUs, 2.28 by the rate of the bare MFMA loop): matrix cores busy for 0.51 of the cycles, 1,015 TFLOP/s =
+// 0.42 of that loop's rate.  Over 128 experts (2,048 Zipf tokens) the clock falls to 1.6 GHz, and a tile of one 16-row
+// block takes 55 % of a full one's time for a quarter of its MFMAs: it waits for its loads instead.
+// The weights, their scales and the row addresses requested side by side, and an epilogue on the hardware exponential,
+// block maxima of one instruction per step and shared conversions: 2,048 tokens 665 -> 630 us, 23 tokens 191 -> 182.
 //
 // gate_up + bias + clamped SwiGLU on the block-scaled MFMA: tile i, column group y (128 intermediate columns).
 // Wave w owns intermediate blocks jb, jb + 1 (jb = 8 y + 2 w) and reads their gate rows (blocks jb, jb + 1) and up
