@@ -600,7 +600,7 @@ NA_DEVICE void xcd_tile(int b, int& tile, int& col) {
 // MFMAs, 11,300 of epilogue (32 activations per lane).  The clock is 1.92 GHz under this load (2.2 with one workgroup on
 // a third of the CUs, 2.28 by the rate of the bare MFMA loop): matrix cores busy for 0.51 of the cycles, 1,015 TFLOP/s =
 // 0.42 of that loop's rate.  Over 128 experts (2,048 Zipf tokens) the clock falls to 1.6 GHz, and a tile of one 16-row
-// block takes 55 % of a full one's time for a quarter of its MFMAs: it waits for its loads instead.
+// block takes 55 % of a full one's time for a quarter of its MFMAs.
 // The weights, their scales and the row addresses requested side by side, and an epilogue on the hardware exponential,
 // block maxima of one instruction per step and shared conversions: 2,048 tokens 665 -> 630 us, 23 tokens 191 -> 182.
 //
