@@ -1,7 +1,7 @@
 """The GEMM entry points (plain and grouped, raw and PS4 scales) at the ends of the E8M0 range, against products formed
 in 64 bits from the codes and scale bytes: bytes 0 .. 2 (weights below bf16's normal range), 253 and 254 (weights past
 bf16's largest value, whose products with small x are finite), 255 (NaN), side by side within a k-tile and within a row
-block; x that is subnormal, infinite or NaN.
+block; x that is subnormal, infinite or NaN.  The t950 layout gives the raw layout's bits.
 
 Bar, per element: one bf16 rounding (at most 2^-8 of the value) of the exact product, and fp32 accumulation of 2,880
 exact products, each added in at most four equal parts: below 4 x 2 x 2,880 x 2^-24 of the sum of their magnitudes.
@@ -99,3 +99,39 @@ def test_gemm_scale_range(name):
         assert worst <= 1.0, (name, m, worst)
         checked += int(ok.sum())
     assert checked > 3 * N_ROWS, (name, checked)
+
+
+@pytest.mark.parametrize("high", [False, True])
+def test_gemm_t950_equals_raw(high):
+    """The C entry points over a t950 pool (layout 2): the raw pool's bits, with the model's scale bytes and with bytes
+    252 .. 254 in every seventh row; two slots, gate_up and down, full and short tiles, plain and grouped."""
+    import torch
+    from neural_amd import _native as N
+    from neural_amd import tiles
+    from neural_amd.moe.layout import GPTOSS_LAYOUT, GPTOSS_LAYOUT_T950, mxfp4_pool_views
+    from neural_amd.q80 import mxfp4_kernels as mk
+    rng = np.random.default_rng(40 + high)
+    slots = np.stack([synth.slot_raw(rng) for _ in range(2)])
+    if high:
+        sc = slots[:, synth.CODE_BYTES:].reshape(2, -1, GK)
+        sc[:, ::7] = rng.integers(252, 255, sc[:, ::7].shape, dtype=np.uint8)
+    raw = torch.from_numpy(slots).cuda()
+    t950 = torch.empty(2, GPTOSS_LAYOUT_T950.slot_bytes, dtype=torch.uint8, device="cuda")
+    tiles.repack_to_t950(raw, t950)
+    gb, db, gs, ds = mxfp4_pool_views(raw, GPTOSS_LAYOUT)
+    x = (synth.bf16_normal(rng, (83, K)).float() * (2.0 ** -100 if high else 1.0)).to(torch.bfloat16).cuda()
+    sl = torch.tensor([1, 0], dtype=torch.int64, device="cuda")
+    for blocks, scales, off, n in ((gb, gs, 0, 5760), (db, ds, 360 * 24576, 2880)):
+        print(f"case gemm t950 n={n} high={high}", flush=True)
+        want = mk.mxfp4_gemm(x, blocks, scales, sl)
+        assert torch.isfinite(want).all()
+        base, s = t950.data_ptr() + off, N.stream(x.device)
+        got = torch.full_like(want, 7.0)
+        N.call("na_mxfp4_gemm", x.data_ptr(), 83, K, base, t950.stride(0), None, 0, 2, sl.data_ptr(), 2, got.data_ptr(), n,
+               s)
+        assert torch.equal(got, want)
+        out = torch.full_like(want, 7.0)
+        plan = mk.GroupedGemmPlan([(x, 1, out[0]), (x, 0, out[1])])
+        N.call("na_mxfp4_gemm_grouped", base, t950.stride(0), None, 0, 2, plan.metadata.data_ptr(), plan.ntiles,
+               plan.block_m, n, K, s)
+        assert torch.equal(out, want)
